@@ -272,7 +272,7 @@ int32_t shwfs_centroids_corr(const float* d_img, int32_t size, const int32_t* d_
  * d_ampl_out = |F| and phase d_phase_out = arg(F) / scale ([npup^2] each).
  * Passed as d_pupil / d_phase of shwfs_sh_comp_image (with d_pupil_unit NULL)
  * they give the spot field F * exp(-i offset).  d_work: [2 * n * npup] floats
- * (complex n x npup rows).  Replaces the field-stop branch of
+ * of scratch.  Replaces the field-stop branch of
  * SutraWfsSH::comp_generic (libsutra/src.cpp/sutra_wfs_sh.cpp:366-391:
  * fsamplipup_krnl, CarmaFFT, submask_krnl, CarmaFFT, fillcamplipup from the
  * focal field, libsutra/src.cu/sutra_wfs.cu:87-181, 1868-1888).
