@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kDmThreads) void sh_image_dft_mlp_kernel(ImageParam
     T.x[k * mlp::SX + c] = (__bf16)(v[e] * M.xs);
   }
   // starts with a barrier
-  mlp::tile_forward<kDmTile, mlp::Fp32Weights, false>(M.params, mlp::Fp32Weights{M.params}, T,
+  mlp::tile_forward<kDmTile>(M.params, mlp::Fp32Weights{M.params}, T,
                                                       tid);
   for (int k = wave; k < rows; k += kDmWaves)
     mlp::spot_slopes(spots[k * 64 + lane], lane, s0 + k, P.nvalid, T.y[k * mlp::NOUT],

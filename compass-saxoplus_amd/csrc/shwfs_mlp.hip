@@ -3,13 +3,11 @@
 // FP32 accumulation, FP32 master weights and Adam.  No counterpart in the
 // reference (a new centroider type next to libsutra's CoG family).
 //
-// One workgroup = 4 waves = a tile of 32 samples.  Forward:
+// Inference: one workgroup = 4 waves = a tile of 32 samples:
 //   Z1 = X W1^T + b1 (MFMA), H1 = gelu(Z1); Z2 = H1 W2^T + b2 (MFMA),
 //   H2 = gelu(Z2); Y = H2 W3^T + b3 (VALU, 2 outputs)
-// Backward of the mean squared error (dY = 2 (Y - T) / (2 n)):
-//   dW3 = dY^T H2 (VALU); dZ2 = (dY W3) * gelu'(Z2); dW2 = dZ2^T H1 (MFMA);
-//   dH1 = dZ2 W2 (MFMA, W2^T copy); dZ1 = dH1 * gelu'(Z1); dW1 = dZ1^T X (MFMA)
-// Weight gradients of the tiles are summed with float atomics.
+// Loss and gradient of the mean squared error (dY = 2 (Y - T) / (2 n)): see
+// mlp_grad_kernel.
 #include <cmath>
 
 #include "shwfs_device.hpp"
@@ -26,20 +24,16 @@ constexpr int TS = 32;          // samples per tile
 constexpr int TPB = 256;        // 4 waves
 using Lds = mlp::Lds<TS>;
 constexpr size_t LDS_BYTES = Lds::bytes();
-// work buffer: bf16 copies W1 (128x64), W2 (128x128), W2^T (128x128)
+// work buffer: bf16 copies of W1 and W2 (inference), or W1, W2 and W2^T as
+// MFMA operands, then the workgroups' partial gradients (gradient)
 constexpr size_t WORK_ELEMS = (size_t)NH * NIN + 2 * (size_t)NH * NH;
 
 // X tile of samples row0 .. row0+TS-1 (rows >= rows_valid zero) -> bf16 in LDS.
-__device__ void load_rows(const float* __restrict__ x, const int* __restrict__ index, long row0,
-                          int rows_valid, float x_scale, const Lds& L) {
+__device__ void load_rows(const float* __restrict__ x, long row0, int rows_valid, float x_scale,
+                          const Lds& L) {
   for (int i = threadIdx.x; i < TS * NIN; i += TPB) {
     const int s = i / NIN, c = i % NIN;
-    float v = 0.0f;
-    if (s < rows_valid) {
-      const long r = index ? (long)index[row0 + s] : row0 + s;
-      v = x[r * NIN + c] * x_scale;
-    }
-    L.x[s * SX + c] = (__bf16)v;
+    L.x[s * SX + c] = (__bf16)(s < rows_valid ? x[(row0 + s) * NIN + c] * x_scale : 0.0f);
   }
 }
 
@@ -47,163 +41,418 @@ __global__ __launch_bounds__(TPB) void mlp_prepare_kernel(const float* __restric
                                                           __bf16* __restrict__ work) {
   __bf16* W1b = work;
   __bf16* W2b = W1b + NH * NIN;
-  __bf16* W2t = W2b + NH * NH;
   for (int i = blockIdx.x * TPB + threadIdx.x; i < NH * NH; i += gridDim.x * TPB) {
     if (i < NH * NIN) W1b[i] = (__bf16)P[OW1 + i];
-    const int r = i / NH, c = i % NH;
-    const __bf16 v = (__bf16)P[OW2 + i];
-    W2b[i] = v;
-    W2t[c * NH + r] = v;
+    W2b[i] = (__bf16)P[OW2 + i];
   }
 }
 
-template <bool TRAIN>
 __global__ __launch_bounds__(TPB) void mlp_tile_kernel(const float* __restrict__ P,
                                                        const __bf16* __restrict__ work,
-                                                       const float* __restrict__ x,
-                                                       const float* __restrict__ t,
-                                                       const int* __restrict__ index, long n,
-                                                       float x_scale, float t_scale,
-                                                       float* __restrict__ y,
-                                                       float* __restrict__ grad,
-                                                       float* __restrict__ loss) {
+                                                       const float* __restrict__ x, long n,
+                                                       float x_scale, float* __restrict__ y) {
   extern __shared__ char smem_raw[];
   const Lds L(smem_raw);
   const __bf16* W1b = work;
   const __bf16* W2b = W1b + NH * NIN;
-  const __bf16* W2t = W2b + NH * NH;
   const long row0 = (long)blockIdx.x * TS;
   const int rows = (int)((n - row0) < TS ? (n - row0) : TS);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  load_rows(x, index, row0, rows, x_scale, L);
-  mlp::tile_forward<TS, Bf16Weights, TRAIN>(P, Bf16Weights{W1b, W2b}, L, (int)threadIdx.x);
-  if constexpr (!TRAIN) {
-    if (tid < rows * NOUT) y[(row0 + tid / NOUT) * NOUT + tid % NOUT] = L.y[tid];
-    return;
-  } else {
-    // ---- loss and dY = 2 (Y - T) / (n * NOUT)
-    float part = 0.0f;
-    if (tid < TS * NOUT) {
-      const int s = tid / NOUT, o = tid % NOUT;
-      float d = 0.0f;
-      if (s < rows) {
-        const long r = index ? (long)index[row0 + s] : row0 + s;
-        d = L.y[tid] - t[r * NOUT + o] * t_scale;
-      }
-      part = d * d;
-      L.dy[tid] = 2.0f * d / (float)(n * NOUT);
-    }
-    part = wave_sum(part);
-    if (lane == 0 && w == 0) atomicAdd(loss, part / (float)(n * NOUT));
-    __syncthreads();
-    // ---- dW3, db3 (thread = (o, k)), and dZ2 = (dY W3) * gelu'(Z2) in place
-    {
-      const int o = tid / NH, k = tid % NH;  // TPB == NOUT * NH
-      float g = 0.0f, gb = 0.0f;
-      for (int s = 0; s < TS; ++s) {
-        g += L.dy[s * NOUT + o] * gelu(L.z2[s * SZ + k]);
-        gb += L.dy[s * NOUT + o];
-      }
-      atomicAdd(&grad[OW3 + o * NH + k], g);
-      if (k == 0) atomicAdd(&grad[OB3 + o], gb);
-    }
-    __syncthreads();
-    for (int i = tid; i < TS * NH; i += TPB) {
-      const int s = i / NH, k = i % NH;
-      float dh = 0.0f;
-#pragma unroll
-      for (int o = 0; o < NOUT; ++o) dh += L.dy[s * NOUT + o] * P[OW3 + o * NH + k];
-      const float dz = dh * gelu_grad(L.z2[s * SZ + k]);
-      L.z2[s * SZ + k] = dz;
-      L.h2[s * SH + k] = (__bf16)dz;
-    }
-    __syncthreads();
-    // db2
-    if (tid < NH) {
-      float gb = 0.0f;
-      for (int s = 0; s < TS; ++s) gb += L.z2[s * SZ + tid];
-      atomicAdd(&grad[OB2 + tid], gb);
-    }
-    // ---- dW2 (n2 x n1) = dZ2^T H1: m-tiles (n2) 2w, 2w+1; all 8 n-tiles (n1); K = TS
-    {
-      bf16x8 bfr[NH / 16];
-#pragma unroll
-      for (int nj = 0; nj < NH / 16; ++nj)
-        bfr[nj] = ld8s(L.h1 + (8 * (lane >> 4)) * SH + 16 * nj + (lane & 15), SH);
-#pragma unroll
-      for (int mm = 0; mm < 2; ++mm) {
-        const int mi = 2 * w + mm;
-        const bf16x8 a = ld8s(L.h2 + (8 * (lane >> 4)) * SH + 16 * mi + (lane & 15), SH);
-#pragma unroll
-        for (int nj = 0; nj < NH / 16; ++nj) {
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-          acc = mfma_bf16(a, bfr[nj], acc);
-          const int col = 16 * nj + (lane & 15);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int row = 16 * mi + 4 * (lane >> 4) + v;
-            atomicAdd(&grad[OW2 + row * NH + col], acc[v]);
-          }
-        }
-      }
-    }
-    __syncthreads();  // h1 is overwritten below
-    // ---- dH1 = dZ2 W2 (B from the W2^T copy); dZ1 = dH1 * gelu'(Z1) in place
-#pragma unroll
-    for (int mi = 0; mi < TS / 16; ++mi)
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const int nj = 2 * w + jj;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < NH / 32; ++ks) {
-          const bf16x8 a = ld8(L.h2 + (16 * mi + (lane & 15)) * SH + 32 * ks + 8 * (lane >> 4));
-          const bf16x8 b = ld8(W2t + (16 * nj + (lane & 15)) * NH + 32 * ks + 8 * (lane >> 4));
-          acc = mfma_bf16(a, b, acc);
-        }
-        const int col = 16 * nj + (lane & 15);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = 16 * mi + 4 * (lane >> 4) + v;
-          const float dz = acc[v] * gelu_grad(L.z1[row * SZ + col]);
-          L.z1[row * SZ + col] = dz;
-          L.h1[row * SH + col] = (__bf16)dz;
-        }
-      }
-    __syncthreads();
-    if (tid < NH) {
-      float gb = 0.0f;
-      for (int s = 0; s < TS; ++s) gb += L.z1[s * SZ + tid];
-      atomicAdd(&grad[OB1 + tid], gb);
-    }
-    // ---- dW1 (n1 x in) = dZ1^T X: m-tiles 2w, 2w+1 (n1), 4 n-tiles (in), K = TS
-    {
-      bf16x8 bfr[NIN / 16];
-#pragma unroll
-      for (int nj = 0; nj < NIN / 16; ++nj)
-        bfr[nj] = ld8s(L.x + (8 * (lane >> 4)) * SX + 16 * nj + (lane & 15), SX);
-#pragma unroll
-      for (int mm = 0; mm < 2; ++mm) {
-        const int mi = 2 * w + mm;
-        const bf16x8 a = ld8s(L.h1 + (8 * (lane >> 4)) * SH + 16 * mi + (lane & 15), SH);
-#pragma unroll
-        for (int nj = 0; nj < NIN / 16; ++nj) {
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-          acc = mfma_bf16(a, bfr[nj], acc);
-          const int col = 16 * nj + (lane & 15);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int row = 16 * mi + 4 * (lane >> 4) + v;
-            atomicAdd(&grad[OW1 + row * NIN + col], acc[v]);
-          }
-        }
-      }
-    }
-  }
+  const int tid = threadIdx.x;
+  load_rows(x, row0, rows, x_scale, L);
+  mlp::tile_forward<TS>(P, Bf16Weights{W1b, W2b}, L, tid);
+  if (tid < rows * NOUT) y[(row0 + tid / NOUT) * NOUT + tid % NOUT] = L.y[tid];
 }
 
-__global__ __launch_bounds__(TPB) void mlp_zero_kernel(float* __restrict__ a, int n) {
-  for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) a[i] = 0.0f;
+// ---- loss and gradient ------------------------------------------------------
+// Every product is taken transposed (hidden units as rows, samples as
+// columns), so that a layer's accumulators are the next product's B operand as
+// they stand: lane j + 16 g of a 16 x 16 tile holds units 16 mt + 4 g + v (v <
+// 4) of sample j, two tiles fill the eight slots of a K step, and the weights
+// are laid out in that order of K (train_weights).  One wave takes 16 samples
+// through the whole network and back with no exchange:
+//   Z1^T = W1 X^T, Z2^T = W2 H1^T, dZ2 = (W3^T dY) gelu'(Z2),
+//   dZ1^T = (W2^T dZ2^T) gelu'(Z1).
+// The weight gradients contract over the samples: H1, X and dZ go to LDS once,
+// samples fastest, and each of the eight waves accumulates 16 rows of dW2 and
+// dW1 over all 128 samples of the step; the biases' and the last layer's
+// gradients are summed over the 16 lanes of a row (row_reduce16).  A workgroup
+// keeps its sums in registers over all of its steps and adds them to the
+// gradient once.
+// (The earlier kernel added 24,962 floats by atomics for every 32 samples,
+// evaluated tanhf four times per hidden unit and read its transposed operands
+// two bytes at a time: 235 us at 65,536 samples.  This one takes 39 us and the
+// sum 6; the bound is the 1,700 VALU instructions of a wave's step, two waves
+// per SIMD.)
+constexpr int kGradWaves = 8;
+constexpr int kGradThreads = 64 * kGradWaves;
+constexpr int kGradStep = 16 * kGradWaves;  // samples of a step
+constexpr int kGradMaxGroups = 256;         // one workgroup per CU (149 KiB of LDS)
+// Up to kGradAtomicGroups workgroups add their sums to the gradient by
+// atomics; more of them store partial gradients that a second kernel sums.
+// Whole calls at 32,768 samples (256 workgroups): 75 us with atomics, 56 with
+// partial sums; at 4,096 (32 workgroups) 45.7 and 44.8: no gain for the work
+// space there.
+constexpr int kGradAtomicGroups = 32;
+constexpr int kGradSlot = NPARAM + 2;       // partial gradient, loss, padding (16-byte rows)
+constexpr int kGradSplit = 8;               // workgroups that share the sum of an element
+constexpr int SS = kGradStep + 8;           // LDS row of samples (16-byte aligned rows)
+constexpr int kFragW1 = NH * NIN, kFragW2 = NH * NH;
+constexpr size_t GRAD_LDS = 2 * sizeof(__bf16) * (size_t)kFragW2 +
+                            sizeof(__bf16) * (size_t)SS * (2 * NH + NIN) +
+                            sizeof(float) * (size_t)(8 * NH + 4);
+
+// The weights as A operands (element e of lane l of fragment (mt, ks) at
+// ((mt KS + ks) 64 + l) 8 + e), K in the order above for W2 and W2^T; and the
+// zeroed gradient and loss.
+__global__ __launch_bounds__(TPB) void mlp_prepare_grad_kernel(const float* __restrict__ P,
+                                                               __bf16* __restrict__ work,
+                                                               float* __restrict__ grad,
+                                                               float* __restrict__ loss) {
+  __bf16* W1f = work;
+  __bf16* W2f = W1f + kFragW1;
+  __bf16* W2tf = W2f + kFragW2;
+  for (int i = blockIdx.x * TPB + threadIdx.x; i < NPARAM; i += gridDim.x * TPB) {
+    const int e = i & 7, l = (i >> 3) & 63, f = i >> 9;
+    const int row = l & 15, g = l >> 4;
+    if (i < kFragW1) W1f[i] = (__bf16)P[OW1 + (16 * (f >> 1) + row) * NIN + 32 * (f & 1) + 8 * g + e];
+    if (i < kFragW2) {
+      const int m = 16 * (f >> 2) + row, k = 32 * (f & 3) + 16 * (e >> 2) + 4 * g + (e & 3);
+      W2f[i] = (__bf16)P[OW2 + m * NH + k];
+      W2tf[i] = (__bf16)P[OW2 + k * NH + m];
+    }
+    grad[i] = 0.0f;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) loss[0] = 0.0f;
+}
+
+// gelu(z) and gelu'(z) from one exponential: with s = 1 / (1 + exp(-2 u)), u =
+// c (z + 0.044715 z^3), (1 + tanh u) / 2 = s and (1 - tanh^2 u) / 4 = s (1 - s).
+// Relative error of s about 3e-7 for every z (1 + tanhf loses its relative
+// accuracy below z = 0).
+__device__ __forceinline__ void gelu_both(float z, float& g, float& dg) {
+  constexpr float k2 = 2.0f * kGeluC, kA = 0.044715f, kLog2e = 1.44269504088896341f;
+  const float z2 = z * z;
+  const float w = z * fmaf(k2 * kA, z2, k2);  // 2 u
+  const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2e * w));
+  g = z * s;
+  dg = fmaf(g * (1.0f - s), fmaf(3.0f * k2 * kA, z2, k2), s);
+}
+
+// Sums over the 16 lanes of a row of the 16 values v: lane j receives the
+// total of value row_reduce16_index(j).  Each step keeps half of the values in
+// half of the lanes (15 adds, where 16 row sums take 64).
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row_reduce16(const float (&v)[16], int lane) {
+  float a[8], b[4], c[2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const bool up = (lane & 8) != 0;
+    a[i] = (up ? v[2 * i + 1] : v[2 * i]) + dpp_move<0x140>(up ? v[2 * i] : v[2 * i + 1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bool up = (lane & 4) != 0;
+    b[i] = (up ? a[2 * i + 1] : a[2 * i]) + dpp_move<0x141>(up ? a[2 * i] : a[2 * i + 1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bool up = (lane & 2) != 0;
+    c[i] = (up ? b[2 * i + 1] : b[2 * i]) + dpp_move<0x1B>(up ? b[2 * i] : b[2 * i + 1]);
+  }
+  const bool up = (lane & 1) != 0;
+  return (up ? c[1] : c[0]) + dpp_move<0xB1>(up ? c[0] : c[1]);
+}
+__device__ __forceinline__ int row_reduce16_index(int lane) {
+  return ((lane >> 3) & 1) | ((lane >> 1) & 2) | ((lane << 1) & 4) | ((lane << 3) & 8);
+}
+
+// 16-byte reads of caller memory (dword alignment is enough)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4u*>(p); }
+__device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+__device__ __forceinline__ bf16x8 pack8(const f32x4& lo, const f32x4& hi) {
+  bf16x8 r;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    r[v] = (__bf16)lo[v];
+    r[4 + v] = (__bf16)hi[v];
+  }
+  return r;
+}
+
+// Units 32 ks + 16 (e >> 2) + 4 g + (e & 3) of sample col to rows of LDS; o =
+// 4 g SS + col, made opaque here so that one address register serves the 32
+// constant offsets (32 hoisted addresses spill).
+__device__ __forceinline__ void store_units(__bf16* t, const bf16x8 (&f)[4], int o) {
+  asm volatile("" : "+v"(o));
+  __bf16* q = t + o;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[(32 * ks + 16 * (e >> 2) + (e & 3)) * SS] = f[ks][e];
+}
+
+// Sums the partial gradients: element (blockIdx.x, thread) of every
+// kGradSplit-th workgroup's slot.
+__global__ __launch_bounds__(TPB) void mlp_grad_sum_kernel(const float* __restrict__ part,
+                                                           int groups, float* __restrict__ grad,
+                                                           float* __restrict__ loss) {
+  const int i = blockIdx.x * TPB + threadIdx.x;
+  if (i > NPARAM) return;
+  float acc = 0.0f;
+#pragma unroll 8
+  for (int k = blockIdx.y; k < groups; k += kGradSplit) acc += part[(size_t)k * kGradSlot + i];
+  atomicAdd(i < NPARAM ? &grad[i] : loss, acc);
+}
+
+// PART: partial gradients to `grad` (kGradSlot floats per workgroup, the loss
+// after the parameters) instead of atomics to the gradient and the loss.
+template <bool PART>
+__global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void mlp_grad_kernel(const float* __restrict__ P, const __bf16* __restrict__ work,
+                     const float* __restrict__ x, const float* __restrict__ t,
+                     const int* __restrict__ index, long n, float x_scale, float t_scale,
+                     float* __restrict__ grad, float* __restrict__ loss) {
+  extern __shared__ __align__(16) char smem_raw[];
+  __bf16* sW2 = reinterpret_cast<__bf16*>(smem_raw);  // W2 fragments
+  __bf16* sW2t = sW2 + kFragW2;                       // W2^T fragments
+  __bf16* sH = sW2t + kFragW2;                        // H1 [unit][sample]
+  __bf16* sD = sH + (size_t)NH * SS;                  // dZ2, then dZ1 [unit][sample]
+  __bf16* sX = sD + (size_t)NH * SS;                  // X [input][sample]
+  float* sB1 = reinterpret_cast<float*>(sX + (size_t)NIN * SS);  // b1, b2, W3
+  float *sB2 = sB1 + NH, *sW3 = sB2 + NH;
+  float* sum = sW3 + NOUT * NH;  // db1, db2, dW3 (2), db3, loss
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const __bf16* W1f = work;
+  for (int i = tid; i < 2 * kFragW2 / 8; i += kGradThreads)
+    reinterpret_cast<float4*>(sW2)[i] = reinterpret_cast<const float4*>(work + kFragW1)[i];
+  if (tid < NH) {
+    sB1[tid] = P[OB1 + tid];
+    sB2[tid] = P[OB2 + tid];
+    sW3[tid] = P[OW3 + tid];
+    sW3[NH + tid] = P[OW3 + NH + tid];
+  }
+  const float b3[2] = {P[OB3], P[OB3 + 1]};
+  for (int i = tid; i < 4 * NH + 4; i += kGradThreads) sum[i] = 0.0f;
+  __syncthreads();
+
+  f32x4 a2[8], a1[4];  // rows 16 w .. 16 w + 15 of dW2 and dW1
+#pragma unroll
+  for (int k = 0; k < 8; ++k) a2[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a1[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float rb1[2] = {0.f, 0.f}, rb2[2] = {0.f, 0.f}, r3[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+  float rdy[2] = {0.f, 0.f}, rl = 0.0f;
+  const long steps = (n + kGradStep - 1) / kGradStep;
+  const float dscale = 2.0f / (float)(n * NOUT);
+
+  for (long st = blockIdx.x; st < steps; st += gridDim.x) {
+    // W1's operands are read anew in each step (from L1, all together):
+    // hoisted out of the loop they would hold 64 registers
+    int anew = 0;
+    asm volatile("" : "+s"(anew));
+    bf16x8 w1[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) w1[k] = ld8(W1f + anew + (k * 64 + lane) * 8);
+    const int col = 16 * w + j;
+    const long s = st * kGradStep + col;
+    const bool valid = s < n;
+    const long r = valid ? (index ? (long)index[s] : s) : 0;
+    const int units = 4 * g * SS + col;
+    int inputs = 8 * g * SS + col;
+    asm volatile("" : "+v"(inputs));
+    // X^T operand straight from the sample's row
+    bf16x8 xf[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const f32x4 lo = ld4(x + r * NIN + 32 * ks + 8 * g), hi = ld4(x + r * NIN + 32 * ks + 8 * g + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        xf[ks][e] = (__bf16)(valid ? (e < 4 ? lo[e & 3] : hi[e & 3]) * x_scale : 0.0f);
+        sX[inputs + (32 * ks + e) * SS] = xf[ks][e];
+      }
+    }
+    const float t0 = t[r * NOUT] * t_scale, t1 = t[r * NOUT + 1] * t_scale;
+
+    // Z1^T, H1 and gelu'(Z1)
+    bf16x8 h1[4];
+    f32x4 d1[8];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      f32x4 hh[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int mt = 2 * ks + q;
+        f32x4 acc = lds4(sB1 + 16 * mt + 4 * g);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) acc = mfma_bf16(w1[2 * mt + k], xf[k], acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float gv, dv;
+          gelu_both(acc[v], gv, dv);
+          hh[q][v] = gv;
+          d1[mt][v] = dv;
+        }
+      }
+      h1[ks] = pack8(hh[0], hh[1]);
+    }
+    store_units(sH, h1, units);
+
+    // Z2^T, the outputs' partial sums and gelu'(Z2)
+    f32x4 h2[8], d2[8];
+    float y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt) {
+      f32x4 acc = lds4(sB2 + 16 * mt + 4 * g);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc = mfma_bf16(ld8(sW2 + ((mt * 4 + k) * 64 + lane) * 8), h1[k], acc);
+      const f32x4 w0 = lds4(sW3 + 16 * mt + 4 * g);
+      const f32x4 w1 = lds4(sW3 + NH + 16 * mt + 4 * g);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float gv, dv;
+        gelu_both(acc[v], gv, dv);
+        h2[mt][v] = gv;
+        d2[mt][v] = dv;
+        y0 = fmaf(gv, w0[v], y0);
+        y1 = fmaf(gv, w1[v], y1);
+      }
+    }
+    // the sample's outputs: four lane groups hold its units
+    y0 += __shfl_xor(y0, 16);
+    y1 += __shfl_xor(y1, 16);
+    y0 += __shfl_xor(y0, 32);
+    y1 += __shfl_xor(y1, 32);
+    const float e0 = valid ? y0 + b3[0] - t0 : 0.0f, e1 = valid ? y1 + b3[1] - t1 : 0.0f;
+    const float dy0 = dscale * e0, dy1 = dscale * e1;
+    rl += e0 * e0 + e1 * e1;  // the same in the four groups
+    rdy[0] += dy0;
+    rdy[1] += dy1;
+
+    // dW3 sums, dZ2 and its bias sums
+    bf16x8 z2[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {  // tiles 4 h .. 4 h + 3: 16 units of the lane
+      float p0[16], p1[16], pb[16];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int mt = 4 * h + i;
+        const f32x4 w0 = lds4(sW3 + 16 * mt + 4 * g);
+        const f32x4 w1 = lds4(sW3 + NH + 16 * mt + 4 * g);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          p0[4 * i + v] = dy0 * h2[mt][v];
+          p1[4 * i + v] = dy1 * h2[mt][v];
+          d2[mt][v] *= fmaf(dy0, w0[v], dy1 * w1[v]);
+          pb[4 * i + v] = d2[mt][v];
+        }
+      }
+      r3[0][h] += row_reduce16(p0, lane);
+      r3[1][h] += row_reduce16(p1, lane);
+      rb2[h] += row_reduce16(pb, lane);
+      z2[2 * h] = pack8(d2[4 * h], d2[4 * h + 1]);
+      z2[2 * h + 1] = pack8(d2[4 * h + 2], d2[4 * h + 3]);
+    }
+    store_units(sD, z2, units);
+
+    // dZ1^T and its bias sums
+    bf16x8 z1[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float pb[16];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int mt = 4 * h + i;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          acc = mfma_bf16(ld8(sW2t + ((mt * 4 + k) * 64 + lane) * 8), z2[k], acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          d1[mt][v] *= acc[v];
+          pb[4 * i + v] = d1[mt][v];
+        }
+        }
+      rb1[h] += row_reduce16(pb, lane);
+      z1[2 * h] = pack8(d1[4 * h], d1[4 * h + 1]);
+      z1[2 * h + 1] = pack8(d1[4 * h + 2], d1[4 * h + 3]);
+    }
+    __syncthreads();  // H1, dZ2 and X of the step
+    // dW2 rows of this wave: dZ2^T H1
+#pragma unroll
+    for (int ks = 0; ks < kGradStep / 32; ++ks) {
+      const bf16x8 a = ld8(sD + (16 * w + j) * SS + 32 * ks + 8 * g);
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt)
+        a2[nt] = mfma_bf16(a, ld8(sH + (16 * nt + j) * SS + 32 * ks + 8 * g), a2[nt]);
+    }
+    __syncthreads();  // dZ2 read
+    store_units(sD, z1, units);
+    __syncthreads();  // dZ1
+#pragma unroll
+    for (int ks = 0; ks < kGradStep / 32; ++ks) {
+      const bf16x8 a = ld8(sD + (16 * w + j) * SS + 32 * ks + 8 * g);
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt)
+        a1[nt] = mfma_bf16(a, ld8(sX + (16 * nt + j) * SS + 32 * ks + 8 * g), a1[nt]);
+    }
+    __syncthreads();  // the step's rows are read
+  }
+
+  // this workgroup's sums: the waves' bias and last-layer sums through LDS
+  // (value i of half h is unit 64 h + 16 (i >> 2) + 4 g + (i & 3))
+  {
+    const int i = row_reduce16_index(lane);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int u = 64 * h + 16 * (i >> 2) + 4 * g + (i & 3);
+      atomicAdd(&sum[u], rb1[h]);
+      atomicAdd(&sum[NH + u], rb2[h]);
+      atomicAdd(&sum[2 * NH + u], r3[0][h]);
+      atomicAdd(&sum[3 * NH + u], r3[1][h]);
+    }
+    const float l = row_sum(rl), q0 = row_sum(rdy[0]), q1 = row_sum(rdy[1]);
+    if (lane == 0) {
+      atomicAdd(&sum[4 * NH], q0);
+      atomicAdd(&sum[4 * NH + 1], q1);
+      atomicAdd(&sum[4 * NH + 2], l);
+    }
+  }
+  __syncthreads();
+  float* slot = PART ? grad + (size_t)blockIdx.x * kGradSlot : grad;
+  auto emit = [&](int i, float v) {
+    if constexpr (PART)
+      slot[i] = v;
+    else
+      atomicAdd(&slot[i], v);
+  };
+  if (tid < NH) {
+    emit(OB1 + tid, sum[tid]);
+    emit(OB2 + tid, sum[NH + tid]);
+    emit(OW3 + tid, sum[2 * NH + tid]);
+    emit(OW3 + NH + tid, sum[3 * NH + tid]);
+    if (tid < NOUT) emit(OB3 + tid, sum[4 * NH + tid]);
+    if (tid == NOUT) {
+      const float l = sum[4 * NH + 2] / (float)(n * NOUT);
+      if constexpr (PART)
+        slot[NPARAM] = l;
+      else
+        atomicAdd(loss, l);
+    }
+  }
+#pragma unroll
+  for (int nt = 0; nt < 8; ++nt)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) emit(OW2 + (16 * w + 4 * g + v) * NH + 16 * nt + j, a2[nt][v]);
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) emit(OW1 + (16 * w + 4 * g + v) * NIN + 16 * nt + j, a1[nt][v]);
 }
 
 __global__ __launch_bounds__(TPB) void mlp_adam_kernel(float* __restrict__ P, float* __restrict__ G,
@@ -259,7 +508,7 @@ __global__ __launch_bounds__(TPB) void mlp_centroid_kernel(
     const int sl = i / NIN, c = i % NIN;
     L.x[sl * SX + c] = (__bf16)(sl < rows ? pixel(row0 + sl, c) * x_scale : 0.0f);
   }
-  mlp::tile_forward<TS, Bf16Weights, false>(P, Bf16Weights{W1b, W2b}, L, (int)threadIdx.x);
+  mlp::tile_forward<TS>(P, Bf16Weights{W1b, W2b}, L, (int)threadIdx.x);
   // flux and CoG from the raw pixels: one wave per 8 sub-apertures
   for (int k = 0; k < TS / 4; ++k) {
     const int sl = w * (TS / 4) + k;
@@ -296,7 +545,9 @@ using namespace shwfs;
 
 extern "C" {
 
-size_t shwfs_mlp_work_bytes(void) { return WORK_ELEMS * sizeof(__bf16); }
+size_t shwfs_mlp_work_bytes(void) {
+  return WORK_ELEMS * sizeof(__bf16) + sizeof(float) * (size_t)kGradMaxGroups * kGradSlot;
+}
 
 int32_t shwfs_phase_window(const float* d_src, int32_t src_side, int32_t ox, int32_t oy,
                            float gain, float* d_dst, int32_t n, void* stream) {
@@ -328,9 +579,8 @@ int32_t shwfs_mlp_forward(const float* d_params, void* d_work, const float* d_x,
   hipStream_t st = (hipStream_t)stream;
   int32_t rc = prepare(d_params, d_work, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(mlp_tile_kernel<false>, dim3(blocks_for(n)), dim3(TPB), LDS_BYTES, st,
-                     d_params, (const __bf16*)d_work, d_x, nullptr, nullptr, (long)n, x_scale, 1.0f,
-                     d_y, nullptr, nullptr);
+  hipLaunchKernelGGL(mlp_tile_kernel, dim3(blocks_for(n)), dim3(TPB), LDS_BYTES, st, d_params,
+                     (const __bf16*)d_work, d_x, (long)n, x_scale, d_y);
   SHWFS_LAUNCHED("mlp_tile_kernel");
   return SHWFS_OK;
 }
@@ -342,15 +592,24 @@ int32_t shwfs_mlp_loss_grad(const float* d_params, void* d_work, const float* d_
     return fail(SHWFS_ERR_ARG, "mlp_loss_grad: NULL argument");
   if (n <= 0) return fail(SHWFS_ERR_ARG, "mlp_loss_grad: n must be positive");
   hipStream_t st = (hipStream_t)stream;
-  int32_t rc = prepare(d_params, d_work, st);
-  if (rc) return rc;
-  hipLaunchKernelGGL(mlp_zero_kernel, dim3(32), dim3(TPB), 0, st, d_grad, NPARAM);
-  hipLaunchKernelGGL(mlp_zero_kernel, dim3(1), dim3(TPB), 0, st, d_loss, 1);
-  SHWFS_LAUNCHED("mlp_zero_kernel");
-  hipLaunchKernelGGL(mlp_tile_kernel<true>, dim3(blocks_for(n)), dim3(TPB), LDS_BYTES, st,
-                     d_params, (const __bf16*)d_work, d_x, d_t, d_index, (long)n, x_scale, t_scale,
-                     nullptr, d_grad, d_loss);
-  SHWFS_LAUNCHED("mlp_tile_kernel");
+  if (GRAD_LDS > max_lds_per_block())
+    return fail(SHWFS_ERR_UNSUPPORTED, "mlp_loss_grad: LDS footprint exceeds the per-workgroup limit");
+  hipLaunchKernelGGL(mlp_prepare_grad_kernel, dim3((NPARAM + TPB - 1) / TPB), dim3(TPB), 0, st,
+                     d_params, (__bf16*)d_work, d_grad, d_loss);
+  SHWFS_LAUNCHED("mlp_prepare_grad_kernel");
+  const int64_t steps = (n + kGradStep - 1) / kGradStep;
+  const unsigned grid = (unsigned)(steps < kGradMaxGroups ? steps : kGradMaxGroups);
+  float* part = reinterpret_cast<float*>(static_cast<char*>(d_work) + WORK_ELEMS * sizeof(__bf16));
+  const bool atomics = grid <= (unsigned)kGradAtomicGroups;
+  hipLaunchKernelGGL(atomics ? mlp_grad_kernel<false> : mlp_grad_kernel<true>, dim3(grid),
+                     dim3(kGradThreads), GRAD_LDS, st, d_params, (const __bf16*)d_work, d_x, d_t,
+                     d_index, (long)n, x_scale, t_scale, atomics ? d_grad : part, d_loss);
+  SHWFS_LAUNCHED("mlp_grad_kernel");
+  if (!atomics) {
+    hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3((NPARAM + TPB) / TPB, kGradSplit), dim3(TPB), 0,
+                       st, part, (int)grid, d_grad, d_loss);
+    SHWFS_LAUNCHED("mlp_grad_sum_kernel");
+  }
   return SHWFS_OK;
 }
 

@@ -22,37 +22,27 @@ constexpr int OW1 = 0, OB1 = OW1 + NH * NIN, OW2 = OB1 + NH, OB2 = OW2 + NH * NH
               OW3 = OB2 + NH, OB3 = OW3 + NOUT * NH, NPARAM = OB3 + NOUT;
 // LDS row strides (elements), padded against bank conflicts
 constexpr int SX = NIN + 8;  // bf16 X
-constexpr int SZ = NH + 4;   // fp32 Z1 / Z2
-constexpr int SH = NH + 8;   // bf16 H1 / H2
+constexpr int SZ = NH + 4;   // fp32 gelu(Z2)
+constexpr int SH = NH + 8;   // bf16 H1
 
 // LDS of a tile of TS samples.
 template <int TS>
 struct Lds {
   __bf16* x;   // [TS][SX]
-  float* z1;   // [TS][SZ]   z1, later dZ1
-  float* z2;   // [TS][SZ]   z2, later dZ2
-  __bf16* h1;  // [TS][SH]   gelu(z1), later dZ1 (bf16)
-  __bf16* h2;  // [TS][SH]   gelu(z2), later dZ2 (bf16)
+  float* g2;   // [TS][SZ]   gelu(z2)
+  __bf16* h1;  // [TS][SH]   gelu(z1)
   float* y;    // [TS][NOUT]
-  float* dy;   // [TS][NOUT]
   static constexpr size_t bytes() {
-    return (size_t)TS * SX * 2 + 2 * (size_t)TS * SZ * 4 + 2 * (size_t)TS * SH * 2 +
-           (size_t)TS * NOUT * 4 * 2;
+    return (size_t)TS * SX * 2 + (size_t)TS * SZ * 4 + (size_t)TS * SH * 2 + (size_t)TS * NOUT * 4;
   }
   __device__ explicit Lds(char* base) {
     x = (__bf16*)base;
     base += (size_t)TS * SX * 2;
-    z1 = (float*)base;
-    base += (size_t)TS * SZ * 4;
-    z2 = (float*)base;
+    g2 = (float*)base;
     base += (size_t)TS * SZ * 4;
     h1 = (__bf16*)base;
     base += (size_t)TS * SH * 2;
-    h2 = (__bf16*)base;
-    base += (size_t)TS * SH * 2;
     y = (float*)base;
-    base += (size_t)TS * NOUT * 4;
-    dy = (float*)base;
   }
 };
 
@@ -60,21 +50,9 @@ constexpr float kGeluC = 0.7978845608028654f;  // sqrt(2 / pi)
 __device__ __forceinline__ float gelu(float z) {
   return 0.5f * z * (1.0f + tanhf(kGeluC * (z + 0.044715f * z * z * z)));
 }
-__device__ __forceinline__ float gelu_grad(float z) {
-  const float t = tanhf(kGeluC * (z + 0.044715f * z * z * z));
-  return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * kGeluC * (1.0f + 3.0f * 0.044715f * z * z);
-}
 
 // 8 consecutive bf16 of a row (16-byte aligned)
 __device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
-// 8 bf16 at stride `st` (column of a row-major array)
-__device__ __forceinline__ bf16x8 ld8s(const __bf16* p, int st) {
-  bf16x8 v;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = p[e * st];
-  return v;
-}
-
 // Weight operands from bf16 copies of W1 and W2 (the training and
 // stand-alone inference kernels, which convert them once per launch).
 struct Bf16Weights {
@@ -106,10 +84,8 @@ struct Fp32Weights {
 // 2w+1 of each layer), four lanes per output the last layer.  The
 // value of a sample does not depend on TS or on the other samples of the
 // tile.  tid: the thread index.
-// KEEP_Z: z1 and z2 keep the pre-activations (the backward pass reads them);
-// otherwise z2 receives gelu(z2) in fp32, which the last layer then reads
-// without computing it again (the same values either way).
-template <int TS, class WS, bool KEEP_Z = true>
+// g2 receives gelu(z2) in fp32, which the last layer reads.
+template <int TS, class WS>
 __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const WS& ws,
                                              const Lds<TS>& L, int tid) {
   const int lane = tid & 63, w = tid >> 6;
@@ -133,7 +109,6 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const 
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * mi + 4 * (lane >> 4) + v;
           const float z = acc[v] + P[OB1 + col];
-          if constexpr (KEEP_Z) L.z1[row * SZ + col] = z;
           L.h1[row * SH + col] = (__bf16)gelu(z);
         }
       }
@@ -159,8 +134,7 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const 
           const int row = 16 * mi + 4 * (lane >> 4) + v;
           const float z = acc[v] + P[OB2 + col];
           const float g = gelu(z);
-          L.z2[row * SZ + col] = KEEP_Z ? z : g;
-          L.h2[row * SH + col] = (__bf16)g;
+          L.g2[row * SZ + col] = g;
         }
       }
   }
@@ -180,8 +154,7 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const 
 #pragma unroll 4
     for (int j = 0; j < NH / PARTS; ++j) {
       const int k = part + PARTS * j;
-      const float z = L.z2[s * SZ + k];
-      acc += (KEEP_Z ? gelu(z) : z) * P[OW3 + o * NH + k];
+      acc += L.g2[s * SZ + k] * P[OW3 + o * NH + k];
     }
 #pragma unroll
     for (int m = 1; m < PARTS; m <<= 1) acc += __shfl_xor(acc, m, PARTS);
