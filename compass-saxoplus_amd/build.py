@@ -23,7 +23,8 @@ ARCH = os.environ.get("SHWFS_OFFLOAD_ARCH", "gfx950")
 
 HIP_SOURCES = ["shwfs_capi.hip", "shwfs_image_fft.hip", "shwfs_image_dft.hip",
                "shwfs_dft_bf16x3_q1.hip", "shwfs_dft_bf16x3_q2.hip", "shwfs_dft_fp16_q1.hip",
-               "shwfs_dft_fp16_q2.hip", "shwfs_batch.hip", "shwfs_batch_quiet.hip",
+               "shwfs_dft_fp16_q2.hip", "shwfs_dft_split.hip",
+               "shwfs_dft_split_ray.hip", "shwfs_batch.hip", "shwfs_batch_quiet.hip",
                "shwfs_batch_noisy.hip", "shwfs_mlp.hip", "shwfs_raytrace.hip",
                "shwfs_image_ext.hip", "shwfs_batch_groups.hip", "shwfs_corr.hip",
                "shwfs_field_stop.hip", "shwfs_lgs.hip", "shwfs_dft_mlp.hip"]

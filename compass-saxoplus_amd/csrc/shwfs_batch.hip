@@ -57,10 +57,11 @@ bool fft_kind(int nfft, int split, int* kind) {
   return true;
 }
 
-bool dft_kind(int nfft, int pdiam, int method, int* kind) {
-  const bool bf = method == SHWFS_METHOD_DFT_BF16X3;
-  if (!bf && method != SHWFS_METHOD_DFT_FP16) return false;
-  const int off = bf ? BK_BF16_16 : BK_FP16_16;
+// prec: an MFMA method or kSplitFp16
+bool dft_kind(int nfft, int pdiam, int prec, int* kind) {
+  if (prec != SHWFS_METHOD_DFT_BF16X3 && prec != SHWFS_METHOD_DFT_FP16 && prec != kSplitFp16)
+    return false;
+  const int off = batch_prec_base(prec);
   if (pdiam <= 16) {
     if (nfft == 16) return *kind = off + 0, true;
     if (nfft == 32) return *kind = off + 1, true;
@@ -85,7 +86,11 @@ int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, hipStream
   const int nfft = g.nfft, pdiam = g.nphase, npix = g.npix;
   int32_t rc = check_geom(&g, tile.method);
   if (rc) return rc;
-  if (tile.method == SHWFS_METHOD_FFT_FP32) {
+  // the FFT method's default tile of a noise-free batch: the products that its
+  // frames take alone (split_fp16_fits); split 1 or 2 names the in-register FFT
+  const bool products = tile.method == SHWFS_METHOD_FFT_FP32 && tile.split == 0 && !b->noisy &&
+                        split_fp16_fits(t.P, nfft);
+  if (tile.method == SHWFS_METHOD_FFT_FP32 && !products) {
     int split = tile.split;
     if (split == 0) split = 2 * pdiam <= nfft ? 2 : 1;
     if (split != 1 && split != 2) return fail(SHWFS_ERR_ARG, "batch: FFT split must be 0, 1 or 2");
@@ -105,13 +110,14 @@ int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, hipStream
     }
     *lds = sizeof(float) * (size_t)t.per_tile * slot;
   } else {
-    if (!dft_kind(nfft, pdiam, tile.method, &t.kind))
+    const int prec = products ? kSplitFp16 : tile.method;
+    if (!dft_kind(nfft, pdiam, prec, &t.kind))
       return fail(SHWFS_ERR_UNSUPPORTED, "batch: DFT stage needs nfft in {16, 32, 64}, pdiam <= 32");
     t.per_tile = kDftTaskSubaps;
     t.nr = dft_register_rebin(t.P);
     const bool gather = t.nr == 0;
     int wf = 0;
-    switch (t.kind - (tile.method == SHWFS_METHOD_DFT_BF16X3 ? BK_BF16_16 : BK_FP16_16)) {
+    switch (t.kind - batch_prec_base(prec)) {
       case 0: wf = subaps_floats<16, 1>(npix, gather, kDftTaskSubaps); break;
       case 1: wf = subaps_floats<32, 1>(npix, gather, kDftTaskSubaps); break;
       case 2: wf = subaps_floats<64, 1>(npix, gather, kDftTaskSubaps); break;
@@ -119,8 +125,10 @@ int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, hipStream
       default: wf = subaps_floats<64, 2>(npix, gather, kDftTaskSubaps); break;
     }
     *lds = sizeof(float) * (size_t)wf;
-    t.wtab = dft_operand_table(nfft, pdiam, tile.method, st);
-    if (!t.wtab) return SHWFS_ERR_HIP;
+    if (!products) {  // (the split-FP16 table is part of the code object)
+      t.wtab = dft_operand_table(nfft, pdiam, tile.method, st);
+      if (!t.wtab) return SHWFS_ERR_HIP;
+    }
   }
   t.ntiles = (g.nvalid + t.per_tile - 1) / t.per_tile;
   *out = t;
@@ -129,16 +137,16 @@ int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, hipStream
 
 // Stage code of a task (stage_code): the FFT with its row split, or the MFMA
 // stage with its window class, full-window flag and register rebin code.
-int task_stage_code(const BatchTask& t, const shwfs_sh_geom& g, int method) {
-  const int n = g.nfft;
-  if (method == SHWFS_METHOD_FFT_FP32) {
+int task_stage_code(const BatchTask& t, const shwfs_sh_geom& g) {
+  const int n = g.nfft, prec = batch_kind_prec(t.kind);
+  if (prec < 0) {
     const int split = (t.kind == BK_FFT16_2 || t.kind == BK_FFT32_2 || t.kind == BK_FFT64_2) ? 2 : 1;
     return stage_code(-1, n, split, false, 0);
   }
   const int q = g.nphase <= 16 ? 1 : 2;
   int nr = dft_register_rebin(t.P);
   if (nr == 4 && dft_half_grid(t.P, n)) nr |= kHalfGrid;
-  return stage_code(method, n, q, g.nphase == 16 * q, nr);
+  return stage_code(prec, n, q, g.nphase == 16 * q, nr);
 }
 
 // Group mode: the tasks' stage codes are three distinct codes in the order of
@@ -153,7 +161,7 @@ bool setup_groups(shwfs_batch* b, std::vector<BatchTask>& tasks, std::vector<dou
   std::vector<int> code(n);
   std::vector<int> distinct;
   for (int i = 0; i < n; ++i) {
-    code[i] = task_stage_code(tasks[i], b->geoms[i], b->tiles[i].method);
+    code[i] = task_stage_code(tasks[i], b->geoms[i]);
     if (std::find(distinct.begin(), distinct.end(), code[i]) == distinct.end())
       distinct.push_back(code[i]);
   }
@@ -172,7 +180,8 @@ bool setup_groups(shwfs_batch* b, std::vector<BatchTask>& tasks, std::vector<dou
     const shwfs_sh_geom& g = b->geoms[i];
     BatchTask& t = tasks[i];
     size_t l = 0;
-    if (b->tiles[i].method == SHWFS_METHOD_FFT_FP32) {
+    const bool fft = batch_kind_prec(t.kind) < 0;
+    if (fft) {
       t.per_tile = 64 / g.nfft;
       const int split = (t.kind == BK_FFT16_2 || t.kind == BK_FFT32_2 || t.kind == BK_FFT64_2) ? 2 : 1;
       int f = 0;
@@ -203,7 +212,7 @@ bool setup_groups(shwfs_batch* b, std::vector<BatchTask>& tasks, std::vector<dou
     t.ntiles = (g.nvalid + t.per_tile - 1) / t.per_tile;
     // the 64-point MFMA stage shares each sub-aperture among the waves of a
     // workgroup: one tile per wave, a quarter sub-aperture each
-    if (b->tiles[i].method != SHWFS_METHOD_FFT_FP32 && g.nfft == 64) t.ntiles = g.nvalid * kDftWaves;
+    if (!fft && g.nfft == 64) t.ntiles = g.nvalid * kDftWaves;
     cost[i] = tile_cost(t, g.nfft);
     wlds = std::max(wlds, l);
   }
@@ -222,7 +231,7 @@ bool setup_groups(shwfs_batch* b, std::vector<BatchTask>& tasks, std::vector<dou
       const int i = order[k];
       if (group[i] != gi) continue;
       first += tasks[i].ntiles;
-      if (b->tiles[i].method != SHWFS_METHOD_FFT_FP32) ga.wtab[gi] = tasks[i].wtab;
+      ga.wtab[gi] = tasks[i].wtab;  // NULL for the FFT and split-FP16
     }
   }
   (void)st;
@@ -250,8 +259,8 @@ int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
   // most kTaskArgs WFS: their parameters travel as kernel arguments): tiles of
   // kDftTaskSubaps sub-apertures, one wave each, kDftWaves waves' LDS slots
   // per workgroup
-  const int m0 = b->tiles[0].method;
-  bool uni = m0 != SHWFS_METHOD_FFT_FP32 && n <= kTaskArgs;
+  const int m0 = batch_kind_prec(tasks[0].kind);
+  bool uni = m0 >= 0 && n <= kTaskArgs;
   for (int i = 0; i < n && uni; ++i) {
     uni = tasks[i].kind == tasks[0].kind && tasks[i].nr == tasks[0].nr &&
           b->geoms[i].nphase == b->geoms[0].nphase;
@@ -262,7 +271,7 @@ int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
       const int npix = b->geoms[i].npix;
       const bool gather = tasks[i].nr == 0;
       int f = 0;
-      switch (tasks[i].kind - (m0 == SHWFS_METHOD_DFT_BF16X3 ? BK_BF16_16 : BK_FP16_16)) {
+      switch (tasks[i].kind - batch_prec_base(m0)) {
         case 0: f = subaps_floats<16, 1>(npix, gather, kDftTaskSubaps); break;
         case 1: f = subaps_floats<32, 1>(npix, gather, kDftTaskSubaps); break;
         case 2: f = subaps_floats<64, 1>(npix, gather, kDftTaskSubaps); break;
@@ -317,7 +326,7 @@ int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
   b->waves = waves;
   int set = 0;
   for (const auto& t : sorted) set |= batch_kind_set(t.kind);
-  b->kind_set = (set == BKS_FFT || set == BKS_BF16 || set == BKS_FP16) ? set : BKS_ALL;
+  b->kind_set = (set & (set - 1)) == 0 ? set : BKS_ALL;  // one set, or all
   b->uni_method = -1;
   if (uni) {
     b->uni_method = m0;
@@ -669,6 +678,7 @@ int32_t shwfs_batch_autotune(shwfs_batch* b, uint32_t method_mask, int32_t reps,
       if (!((method_mask >> m) & 1u) || check_geom(&g, m) != SHWFS_OK) continue;
       if (m == SHWFS_METHOD_FFT_FP32) {
         if (g.nfft != 16 && g.nfft != 32 && g.nfft != 64) continue;
+        if (!b->noisy) cands.push_back(shwfs_batch_tile{m, 0});
         cands.push_back(shwfs_batch_tile{m, 1});
         if (2 * g.nphase <= g.nfft) cands.push_back(shwfs_batch_tile{m, 2});
       } else {

@@ -96,11 +96,15 @@ static int32_t launch_groups(bool noisy, int wpe, const TaskStarts& starts, cons
   if (total <= 0) return SHWFS_OK;
   const int slot = (int)(lds / sizeof(float));
   const dim3 grid((total + kDftWaves - 1) / kDftWaves), block(64 * kDftWaves);
-  if (noisy)  // the noisy kernels keep the 4-wave budget
-    hipLaunchKernelGGL((sh_batch_groups_kernel<S0, S1, S2, true, 4>), grid, block,
-                       lds * kDftWaves, st, starts, args, ntasks, total, ga, slot, frame_base,
-                       frame_off);
-  else if (wpe == 3)
+  if (noisy) {
+    // the noisy kernels keep the 4-wave budget; the split-FP16 stages have none
+    if constexpr (S1::PREC == kSplitFp16)
+      return fail(SHWFS_ERR_ARG, "batch: the split-FP16 stages are noise-free");
+    else
+      hipLaunchKernelGGL((sh_batch_groups_kernel<S0, S1, S2, true, 4>), grid, block,
+                         lds * kDftWaves, st, starts, args, ntasks, total, ga, slot, frame_base,
+                         frame_off);
+  } else if (wpe == 3)
     hipLaunchKernelGGL((sh_batch_groups_kernel<S0, S1, S2, false, 3>), grid, block,
                        lds * kDftWaves, st, starts, args, ntasks, total, ga, slot, frame_base,
                        frame_off);
@@ -126,6 +130,8 @@ using Bf64b = GroupStage<kBf, 64, 2, true, kHalf4>;
 using Fp16a = GroupStage<kFp, 16, 1, false, 2>;
 using Fp32a = GroupStage<kFp, 32, 1, true, kHalf4>;
 using Fp64b = GroupStage<kFp, 64, 2, true, kHalf4>;
+using Sp16a = GroupStage<kSplitFp16, 16, 1, false, 2>;
+using Sp32a = GroupStage<kSplitFp16, 32, 1, true, kHalf4>;
 
 using Launcher = int32_t (*)(bool, int, const TaskStarts&, const TaskArgs&, int, int,
                              const GroupArgs&, size_t, const uint32_t*, uint32_t, hipStream_t);
@@ -145,6 +151,7 @@ const GroupKernel kGroupKernels[] = {
     SHWFS_GK(Fp64b, Fp16a, Fp32a),  // every WFS on FP16
     SHWFS_GK(Fp64b, Bf16a, Bf32a),
     SHWFS_GK(Fp64b, Fft16, Fft32),
+    SHWFS_GK(Fft64, Sp16a, Sp32a),  // every WFS on the FFT method, noise-free
 };
 #undef SHWFS_GK
 

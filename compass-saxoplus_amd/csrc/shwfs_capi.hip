@@ -643,7 +643,8 @@ static int32_t comp_image_on(const shwfs_sh_geom* g, const shwfs_frame_args* f, 
     RayParams r;
     rc = ray_params(f->layers, f->nlayers, g->npup, g->npup, &r);
     if (rc) return rc;
-    return launch_image_fft_ray(p, r, g->nfft, st);
+    return split_fp16_fits(p, g->nfft) ? launch_split_ray(p, r, g->nfft, st)
+                                       : launch_image_fft_ray(p, r, g->nfft, st);
   }
   if (mlp) {
     const shwfs_centroid_args* c = f->centroid;
@@ -653,7 +654,9 @@ static int32_t comp_image_on(const shwfs_sh_geom* g, const shwfs_frame_args* f, 
       return launch_image_dft_mlp(p, m, g->nfft, f->method, st, wtab, bg);
     return launch_image_fft_mlp(p, m, g->nfft, st, bg);
   }
-  if (f->method == SHWFS_METHOD_FFT_FP32) return launch_image_fft(p, g->nfft, st, bg);
+  if (f->method == SHWFS_METHOD_FFT_FP32)
+    return split_fp16_fits(p, g->nfft) ? launch_image_split(p, g->nfft, st)
+                                       : launch_image_fft(p, g->nfft, st, bg);
   return launch_image_dft(p, g->nfft, f->method, st, wtab, bg);
 }
 

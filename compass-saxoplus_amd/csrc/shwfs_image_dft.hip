@@ -44,6 +44,7 @@ int32_t launch_dft_tasks(int method, int nfft, int pdiam, bool full, int nr, boo
   if (method == SHWFS_METHOD_DFT_BF16X3)
     return q1 ? launch_dft_tasks_pq<SHWFS_METHOD_DFT_BF16X3, 1>(SHWFS_ARGS)
               : launch_dft_tasks_pq<SHWFS_METHOD_DFT_BF16X3, 2>(SHWFS_ARGS);
+  if (method == kSplitFp16 && q1) return launch_dft_tasks_pq<kSplitFp16, 1>(SHWFS_ARGS);
 #undef SHWFS_ARGS
   return fail(SHWFS_ERR_ARG, "unknown DFT method");
 }
@@ -57,6 +58,14 @@ int32_t launch_image_dft(const ImageParams& p, int nfft, int method, hipStream_t
   if (method == SHWFS_METHOD_DFT_BF16X3)
     return launch_dft_p<SHWFS_METHOD_DFT_BF16X3>(p, nfft, st, wtab, bg);
   return fail(SHWFS_ERR_ARG, "unknown DFT method");
+}
+
+bool split_fp16_fits(const ImageParams& p, int nfft) {
+  return !(p.noise > -1.0f) && p.tpb == 0 && (nfft == 16 || nfft == 32) && p.pdiam <= 16;
+}
+
+int32_t launch_image_split(const ImageParams& p, int nfft, hipStream_t st) {
+  return launch_dft_pq<kSplitFp16, 1>(p, nfft, st, nullptr, BgParams{});
 }
 
 int32_t build_dft_operand_table(int nfft, int pdiam, int method, void* dst, size_t cap,

@@ -21,9 +21,20 @@
 //     sub-aperture is scaled by a power of two s such that the bound
 //     pdiam * max|E| >= max|G| lands in [2^14, 2^15), and the flux by 1/s^2
 //     (max|E| <= 1 for a window of unit pupil, measured otherwise).
-// The field uses the hardware sine and cosine on the angle in turns (about
-// 1e-6 absolute error): these methods trade accuracy for speed and state their
-// error against the float64 oracle.  Binning, noise, detector image and
+// The field of these two uses the hardware sine and cosine on the angle in
+// turns (about 1e-6 absolute error): they trade accuracy for speed and state
+// their error against the float64 oracle.
+//   * kSplitFp16 (no method of its own: how noise-free frames of
+//     SHWFS_METHOD_FFT_FP32 run, split_fp16_fits): every operand x = hi + lo
+//     (fp16 each, 23 significant bits; the power-of-two scales of FP16 keep lo
+//     in range), hi*hi + hi*lo + lo*hi, 3 MFMA per tile, and the field's
+//     float-exact reduction and polynomials (phase_sincos).  For nfft 16 and
+//     32 with windows of up to 16 points.  Relative error of the spots against
+//     float64 over those shapes: 6-11e-8, the in-register FP32 FFT's 6-11e-8
+//     (80x80, nfft 32: 7.8e-8 against 8.8e-8; 40x40, nfft 16: 8.5 against
+//     8.9e-8).  The FFT is bound by its 1,660 VALU instructions per two
+//     sub-apertures; here the transform is on the matrix cores.
+// Binning, noise, detector image and
 // centroids follow the same definitions as the FFT kernel.
 #pragma once
 
@@ -38,6 +49,16 @@ namespace shwfs {
 // Bit of a compile-time rebin code (rebin factor in bits 0-2) selecting the
 // half-grid 4x4 binning form (dft_half_grid).
 constexpr int kHalfGrid = 8;
+
+// Operand precision of the split-FP16 products (beside the two MFMA methods).
+constexpr int kSplitFp16 = 3;
+// Operands carried as hi + lo; fields scaled by a power of two.
+__host__ __device__ constexpr bool prec_split(int prec) {
+  return prec == SHWFS_METHOD_DFT_BF16X3 || prec == kSplitFp16;
+}
+__host__ __device__ constexpr bool prec_scaled(int prec) {
+  return prec == SHWFS_METHOD_DFT_FP16 || prec == kSplitFp16;
+}
 
 template <int N, int Q>
 struct DftLayout {
@@ -80,6 +101,36 @@ struct Frag<SHWFS_METHOD_DFT_BF16X3> {
   }
 };
 
+template <>
+struct Frag<kSplitFp16> {
+  f16x8 hi, lo;
+};
+
+// The eight slots of an operand.
+template <int PREC>
+__device__ __forceinline__ void frag_set(Frag<PREC>& f, const float (&x)[8]) {
+  if constexpr (PREC == kSplitFp16) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    // x - hi as a mixed-precision multiply-add rounded to fp16 (one
+    // instruction); the factor -1 is hidden from the optimiser, which would
+    // turn it into a conversion, a subtraction and a conversion
+    float m1 = -1.0f;
+    asm("" : "+s"(m1));
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const f16x2 h = __builtin_convertvector((f32x2{x[e], x[e + 1]}), f16x2);
+      f.hi[e] = h.x;
+      f.hi[e + 1] = h.y;
+      f.lo[e] = (_Float16)__builtin_fmaf((float)h.x, m1, x[e]);
+      f.lo[e + 1] = (_Float16)__builtin_fmaf((float)h.y, m1, x[e + 1]);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f.set(e, x[e]);
+  }
+}
+
 __device__ __forceinline__ f32x4 mma(const Frag<SHWFS_METHOD_DFT_FP16>& a,
                                      const Frag<SHWFS_METHOD_DFT_FP16>& b, f32x4 c) {
   return mfma_f16(a.v, b.v, c);
@@ -89,6 +140,12 @@ __device__ __forceinline__ f32x4 mma(const Frag<SHWFS_METHOD_DFT_BF16X3>& a,
   c = mfma_bf16(a.lo, b.hi, c);
   c = mfma_bf16(a.hi, b.lo, c);
   return mfma_bf16(a.hi, b.hi, c);
+}
+__device__ __forceinline__ f32x4 mma(const Frag<kSplitFp16>& a, const Frag<kSplitFp16>& b,
+                                     f32x4 c) {
+  c = mfma_f16(a.lo, b.hi, c);
+  c = mfma_f16(a.hi, b.lo, c);
+  return mfma_f16(a.hi, b.hi, c);
 }
 
 // Contraction slot e of K step ks in lane group g (= lane >> 4) of an
@@ -129,8 +186,40 @@ __device__ __forceinline__ float aw_value(int mt, int ks, int lane, int e) {
 // t = 0.
 template <int Q, int PREC>
 constexpr int table_exp() {
-  return PREC == SHWFS_METHOD_DFT_FP16 ? (Q == 1 ? 10 : 9) : 0;
+  return prec_scaled(PREC) ? (Q == 1 ? 10 : 9) : 0;
 }
+
+// The split-FP16 operand table, computed by the compiler and part of the code
+// object: nothing is allocated or built at run time, so a first frame may be
+// captured.  Element e of lane l of fragment (mt, ks): hi[..][l][e], lo.
+template <int N, int Q>
+struct alignas(16) SplitTable {
+  static constexpr int F = DftLayout<N, Q>::MT * DftLayout<N, Q>::KS;
+  _Float16 v[F][64][2][8];
+  constexpr SplitTable() : v() {
+    constexpr double scale = (double)(1 << table_exp<Q, kSplitFp16>());
+    double c[N] = {};
+    for (int k = 0; k < N; ++k) c[k] = scale * cx_cos2pi(k, N);
+    for (int f = 0; f < F; ++f)
+      for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e) {
+          // aw_value on (mt, ks) = (f / KS, f % KS)
+          const int m = 16 * (f / Q) + (l & 15);
+          const bool row_im = m >= N, col_im = Q == 1 ? e >= 4 : f % Q == 1;
+          const int kx = row_im ? m - N : m;
+          const int x = 4 * (l >> 4) + (e & 3) + (Q == 1 ? 0 : 16 * (e >> 2));
+          const int idx = (kx * x) % N;
+          const double cs = c[idx], sn = c[(idx + N - N / 4) % N];  // cos, sin of 2 pi idx / N
+          // [Wr, -Wi; Wi, Wr] with W = cos - i sin
+          const float w = (float)(row_im == col_im ? cs : (row_im ? -sn : sn));
+          const _Float16 h = (_Float16)w;
+          v[f][l][0][e] = h;
+          v[f][l][1][e] = (_Float16)(w - (float)h);
+        }
+  }
+};
+template <int N, int Q>
+__device__ constexpr SplitTable<N, Q> kSplitTable{};
 
 // The A_W operand (times 2^table_exp) as per-lane fragments, built once per
 // device and kept in a small device table.
@@ -169,6 +258,20 @@ static const Frag<PREC>* wfrag_table(hipStream_t st) {
   return t;
 }
 
+// Fragment f of the operand table t (split-FP16: of the compiled table).
+template <int N, int Q, int PREC>
+__device__ __forceinline__ Frag<PREC> load_frag(const Frag<PREC>* t, int f, int lane) {
+  if constexpr (PREC == kSplitFp16) {
+    Frag<PREC> r;
+    const auto& v = kSplitTable<N, Q>.v[f][lane];
+    r.hi = *reinterpret_cast<const f16x8*>(&v[0][0]);
+    r.lo = *reinterpret_cast<const f16x8*>(&v[1][0]);
+    return r;
+  } else {
+    return t[f * 64 + lane];
+  }
+}
+
 // Source of the A_W fragments: registers (small tables) or the device table
 // (reads that stay in L1/L2).
 template <int N, int Q, int PREC, bool REGS = DftLayout<N, Q>::kAwInRegs>
@@ -179,7 +282,7 @@ struct AwOperand {
 #pragma unroll
     for (int mt = 0; mt < L::MT; ++mt)
 #pragma unroll
-      for (int ks = 0; ks < L::KS; ++ks) f[mt][ks] = t[(mt * L::KS + ks) * 64 + lane];
+      for (int ks = 0; ks < L::KS; ++ks) f[mt][ks] = load_frag<N, Q, PREC>(t, mt * L::KS + ks, lane);
   }
   __device__ __forceinline__ Frag<PREC> get(int mt, int ks) const { return f[mt][ks]; }
 };
@@ -187,9 +290,10 @@ template <int N, int Q, int PREC>
 struct AwOperand<N, Q, PREC, false> {
   using L = DftLayout<N, Q>;
   const Frag<PREC>* t;
-  __device__ __forceinline__ AwOperand(const Frag<PREC>* tab, int lane) : t(tab + lane) {}
+  int lane;
+  __device__ __forceinline__ AwOperand(const Frag<PREC>* tab, int l) : t(tab), lane(l) {}
   __device__ __forceinline__ Frag<PREC> get(int mt, int ks) const {
-    return t[(mt * L::KS + ks) * 64];
+    return load_frag<N, Q, PREC>(t, mt * L::KS + ks, lane);
   }
 };
 
@@ -198,11 +302,8 @@ struct AwOperand<N, Q, PREC, false> {
 template <int PREC>
 __device__ __forceinline__ Frag<PREC> acc_to_operand(const f32x4& X, const f32x4& Y) {
   Frag<PREC> f;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    f.set(v, X[v]);
-    f.set(4 + v, Y[v]);
-  }
+  const float x[8] = {X[0], X[1], X[2], X[3], Y[0], Y[1], Y[2], Y[3]};
+  frag_set(f, x);
   return f;
 }
 
@@ -232,9 +333,9 @@ __device__ __forceinline__ int field_px(int lane, int j) {
 
 typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// The offsets (the same for every window) at the lane's points, as turns:
-// of = -offset / (2 pi).
-template <int N, int Q, bool FULL>
+// The offsets (the same for every window) at the lane's points, as turns: of
+// = -offset / (2 pi); as they are for split-FP16 (phase_sincos).
+template <int N, int Q, int PREC, bool FULL>
 __device__ __forceinline__ void field_offsets(const ImageParams& P, int lane,
                                               float (&of)[Q][FieldIn<Q>::NP]) {
   constexpr int NP = FieldIn<Q>::NP;
@@ -257,8 +358,10 @@ __device__ __forceinline__ void field_offsets(const ImageParams& P, int lane,
         of[ma][j] = P.offsets[(unsigned)(in ? x + y * pdiam : 0)];
       }
     }
+    if constexpr (PREC != kSplitFp16) {
 #pragma unroll
-    for (int j = 0; j < NP; ++j) of[ma][j] = -of[ma][j] * 0.15915494309189533577f;
+      for (int j = 0; j < NP; ++j) of[ma][j] = -of[ma][j] * 0.15915494309189533577f;
+    }
   }
 }
 
@@ -295,6 +398,25 @@ __device__ __forceinline__ void field_load(const ImageParams& P, unsigned win, i
         f.ph[ma][j] =
             *reinterpret_cast<const float*>(reinterpret_cast<const char*>(P.phase) + (g << 2));
       }
+    }
+  }
+}
+
+// The same phases traced through the layers of R (ray_phase; (i0, j0): the
+// window's corner) instead of read from the rendered screen.
+template <int N, int Q, bool FULL>
+__device__ __forceinline__ void field_trace(const RayParams& R, int i0, int j0, int pdiam_rt,
+                                            int lane, FieldIn<Q>& f) {
+  constexpr int NP = FieldIn<Q>::NP;
+  const int pdiam = FULL ? DftLayout<N, Q>::P16 : pdiam_rt;
+#pragma unroll
+  for (int ma = 0; ma < Q; ++ma) {
+    const int y = 16 * ma + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int x = field_px<Q>(lane, j);
+      const bool in = FULL || (x < pdiam && y < pdiam);
+      f.ph[ma][j] = ray_phase(R, i0 + (in ? x : 0), j0 + (in ? y : 0));
     }
   }
 }
@@ -341,11 +463,12 @@ __device__ __forceinline__ void field_amplitude(const ImageParams& P, unsigned w
 
 // Field E = amplitude * exp(i (phase scale - offset)) at the lane's points,
 // as stage A's operand.  The angle is taken in turns, reduced to [0, 1) by
-// v_fract, and fed to the hardware sine and cosine.
+// v_fract, and fed to the hardware sine and cosine; split-FP16 takes
+// phase_sincos.
 // UNIT: a unit-pupil full window (amplitude 1 everywhere: pu is not read).
 // of: the offsets in turns (field_offsets); pu: the amplitude
 // (field_amplitude).
-template <int N, int Q, bool UNIT>
+template <int N, int Q, int PREC, bool UNIT>
 __device__ __forceinline__ void field_eval(const ImageParams& P, int lane, const FieldIn<Q>& f,
                                            const float (&of)[Q][FieldIn<Q>::NP],
                                            const float (&pu)[Q][FieldIn<Q>::NP],
@@ -358,9 +481,13 @@ __device__ __forceinline__ void field_eval(const ImageParams& P, int lane, const
   for (int ma = 0; ma < Q; ++ma)
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
-      const float r = __builtin_amdgcn_fractf(fmaf(f.ph[ma][j], turn_scale, of[ma][j]));
-      er[ma][j] = __builtin_amdgcn_cosf(r);
-      ei[ma][j] = __builtin_amdgcn_sinf(r);
+      if constexpr (PREC == kSplitFp16) {
+        phase_sincos(f.ph[ma][j], P.scale, of[ma][j], ei[ma][j], er[ma][j]);
+      } else {
+        const float r = __builtin_amdgcn_fractf(fmaf(f.ph[ma][j], turn_scale, of[ma][j]));
+        er[ma][j] = __builtin_amdgcn_cosf(r);
+        ei[ma][j] = __builtin_amdgcn_sinf(r);
+      }
       if constexpr (!UNIT) {
         er[ma][j] *= pu[ma][j];
         ei[ma][j] *= pu[ma][j];
@@ -498,12 +625,12 @@ __device__ __forceinline__ void dft_spot(const ImageParams& P, const int lane, f
   int e_total = t;  // G carries 2^e_total
   float ev[Q][Q][8];
   if (FULL && unit) {
-    field_eval<N, Q, FULL>(P, lane, fin, of, of, ev);
+    field_eval<N, Q, PREC, FULL>(P, lane, fin, of, of, ev);
   } else {
     float pu[Q][FieldIn<Q>::NP];
     field_amplitude<N, Q, FULL>(P, win, unit, lane, pu);
-    field_eval<N, Q, false>(P, lane, fin, of, pu, ev);
-    if constexpr (PREC == SHWFS_METHOD_DFT_FP16) {
+    field_eval<N, Q, PREC, false>(P, lane, fin, of, pu, ev);
+    if constexpr (prec_scaled(PREC)) {
       if (!unit) {
         float m = 0.0f;
 #pragma unroll
@@ -530,9 +657,7 @@ __device__ __forceinline__ void dft_spot(const ImageParams& P, const int lane, f
 #pragma unroll
   for (int ma = 0; ma < Q; ++ma)
 #pragma unroll
-    for (int ks = 0; ks < Q; ++ks)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ae[ma][ks].set(e, ev[ma][ks][e]);
+    for (int ks = 0; ks < Q; ++ks) frag_set(ae[ma][ks], ev[ma][ks]);
 
   // ---- stage A: G (rows y, cols (re/im, kx)) = E A_W^T
   constexpr int NTW = L::NTB / PARTS;  // kx blocks of this wave
@@ -619,7 +744,8 @@ __host__ __device__ constexpr bool dft_pair_stage() {
   return N == 16 && Q == 1 && !FULL && NRC >= 0 && (NRC & 7) > 0;
 }
 
-// Offsets (in turns) at the lane's points of its pair row (row = lane & 7).
+// Offsets (as field_offsets) at the lane's points of its pair row (lane & 7).
+template <int PREC>
 __device__ __forceinline__ void field_offsets_pair(const ImageParams& P, int lane,
                                                    float (&of)[1][FieldIn<1>::NP]) {
   const int pdiam = P.pdiam, row = lane & 7;
@@ -629,8 +755,10 @@ __device__ __forceinline__ void field_offsets_pair(const ImageParams& P, int lan
     const bool in = x < pdiam && row < pdiam;
     of[0][j] = P.offsets[(unsigned)(in ? x + row * pdiam : 0)];
   }
+  if constexpr (PREC != kSplitFp16) {
 #pragma unroll
-  for (int j = 0; j < FieldIn<1>::NP; ++j) of[0][j] = -of[0][j] * 0.15915494309189533577f;
+    for (int j = 0; j < FieldIn<1>::NP; ++j) of[0][j] = -of[0][j] * 0.15915494309189533577f;
+  }
 }
 
 // Screen values at the lane's points: window a for rows y < 8, b above.
@@ -672,9 +800,11 @@ __device__ __forceinline__ void field_amplitude_pair(const ImageParams& P, unsig
 
 // Lanes 0-31 of f (lanes 32-63 zero) and lanes 32-63 of f moved to lanes
 // 0-31 (lanes 32-63 zero).  Every lane active.
-__device__ __forceinline__ void split_lane_halves(const Frag<SHWFS_METHOD_DFT_BF16X3>& f,
-                                                  Frag<SHWFS_METHOD_DFT_BF16X3>& lower,
-                                                  Frag<SHWFS_METHOD_DFT_BF16X3>& upper) {
+template <int PREC>
+__device__ __forceinline__ void split_lane_halves(const Frag<PREC>& f, Frag<PREC>& lower,
+                                                  Frag<PREC>& upper) {
+  static_assert(prec_split(PREC), "split_lane_halves: hi + lo operands");
+  using V = decltype(f.hi);
   typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
   const u32x4v h = __builtin_bit_cast(u32x4v, f.hi), l = __builtin_bit_cast(u32x4v, f.lo);
   u32x4v h0, h1, l0, l1;
@@ -688,10 +818,10 @@ __device__ __forceinline__ void split_lane_halves(const Frag<SHWFS_METHOD_DFT_BF
     l0[d] = rl[0];
     l1[d] = rl[1];
   }
-  lower.hi = __builtin_bit_cast(bf16x8, h0);
-  lower.lo = __builtin_bit_cast(bf16x8, l0);
-  upper.hi = __builtin_bit_cast(bf16x8, h1);
-  upper.lo = __builtin_bit_cast(bf16x8, l1);
+  lower.hi = __builtin_bit_cast(V, h0);
+  lower.lo = __builtin_bit_cast(V, l0);
+  upper.hi = __builtin_bit_cast(V, h1);
+  upper.lo = __builtin_bit_cast(V, l1);
 }
 
 __device__ __forceinline__ void split_lane_halves(const Frag<SHWFS_METHOD_DFT_FP16>& f,
@@ -737,11 +867,11 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
   {
     float pu[1][FieldIn<1>::NP];
     field_amplitude_pair(P, win_a, win_b, unit_a, unit_b, lane, pu);
-    field_eval<N, 1, false>(P, lane, fin, of, pu, ev);
+    field_eval<N, 1, PREC, false>(P, lane, fin, of, pu, ev);
   }
   // FP16 field scale of each half (dft_spot's rule on its window alone)
   int e_a = t, e_b = t;
-  if constexpr (PREC == SHWFS_METHOD_DFT_FP16) {
+  if constexpr (prec_scaled(PREC)) {
     if (!unit_a || !unit_b) {  // uniform
       float m = 0.0f;
 #pragma unroll
@@ -758,8 +888,7 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
     }
   }
   F ae;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) ae.set(e, ev[0][0][e]);
+  frag_set(ae, ev[0][0]);
   f32x4 ga[L::MT];
 #pragma unroll
   for (int nt = 0; nt < L::MT; ++nt) {
@@ -791,11 +920,13 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
 // (nr == 0), the moment totals use the 192 doubles after the spot (nr > 0)
 // or at the start, over the dead |F|^2 image (nr == 0).  KEEP: no centroider;
 // the spot-cube values stay in the spot.
-template <int N, int Q, int PREC, bool NOISE, bool FULL, int NRC = -1, bool KEEP = false>
+// RAY: the window's phases are traced through the layers of *ray.
+template <int N, int Q, int PREC, bool NOISE, bool FULL, int NRC = -1, bool KEEP = false,
+          bool RAY = false>
 __device__ __forceinline__ void dft_subap(const ImageParams& P, const int s, const int lane,
                                           float* smem, const int* bm, const int nr_rt,
                                           const AwOperand<N, Q, PREC>& aw,
-                                          unsigned call_add = 0u) {
+                                          unsigned call_add = 0u, const RayParams* ray = nullptr) {
   using L = DftLayout<N, Q>;
   const int nr = NRC >= 0 ? (NRC & 7) : nr_rt;
   SubapScalars pre;
@@ -806,10 +937,13 @@ __device__ __forceinline__ void dft_subap(const ImageParams& P, const int s, con
   const int pdiam = FULL ? L::P16 : P.pdiam;
   const bool unit = unit_window(P, s);
   float of[Q][FieldIn<Q>::NP];
-  field_offsets<N, Q, FULL>(P, lane, of);
+  field_offsets<N, Q, PREC, FULL>(P, lane, of);
   const unsigned win = window_corner(P, s);
   FieldIn<Q> fin;
-  field_load<N, Q, FULL>(P, win, lane, fin);
+  if constexpr (RAY)
+    field_trace<N, Q, FULL>(*ray, P.istart[s], P.jstart[s], P.pdiam, lane, fin);
+  else
+    field_load<N, Q, FULL>(P, win, lane, fin);
   float inten_scale;
   dft_spot<N, Q, PREC, FULL, NRC>(P, lane, smem, bin, bm, nr_rt, aw, fin, of, win, unit,
                                   inten_scale);
@@ -836,7 +970,7 @@ __device__ __forceinline__ void dft_subap_parts(const ImageParams& P, const int 
   const int spot_f = (npix * npix + 3) & ~3;
   const bool unit = unit_window(P, s);
   float of[Q][FieldIn<Q>::NP];
-  field_offsets<N, Q, FULL>(P, lane, of);
+  field_offsets<N, Q, PREC, FULL>(P, lane, of);
   const unsigned win = window_corner(P, s);
   FieldIn<Q> fin;
   field_load<N, Q, FULL>(P, win, lane, fin);
@@ -901,7 +1035,7 @@ __device__ __forceinline__ void dft_subaps(const ImageParams& P, const int s0, c
     // two sub-apertures per stage A (dft_spot_pair); each pair's screen values
     // are loaded while the previous pair is computed
     if constexpr (dft_pair_stage<N, Q, PREC, FULL, NRC>()) {
-      field_offsets_pair(P, lane, of);
+      field_offsets_pair<PREC>(P, lane, of);
       field_load_pair(P, win[0], win[1], lane, fin[0]);
 #pragma unroll
       for (int k = 0; k < SPW; k += 2) {
@@ -918,7 +1052,7 @@ __device__ __forceinline__ void dft_subaps(const ImageParams& P, const int s0, c
       }
     }
   } else {
-    field_offsets<N, Q, FULL>(P, lane, of);
+    field_offsets<N, Q, PREC, FULL>(P, lane, of);
     field_load<N, Q, FULL>(P, win[0], lane, fin[0]);
 #pragma unroll
     for (int k = 0; k < SPW; ++k) {
@@ -1004,6 +1138,30 @@ void sh_image_dft_kernel(ImageParams P, const Frag<PREC>* wtab, BgParams bg) {
   }
 }
 
+// The split-FP16 spot kernel with the guide-star raytrace in its field stage
+// (noise-free): the npup^2 screen is neither written nor read back.
+template <int N, int Q, bool FULL, int NR>
+__global__ __launch_bounds__(64 * kDftWaves)
+void sh_image_dft_ray_kernel(ImageParams P, RayParams Ry) {
+  constexpr int nr = NR & 7;
+  using L = DftLayout<N, Q>;
+  extern __shared__ float smem[];
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int WF = L::wave_floats(P.npix, nr == 0);
+  int* s_binmap = (int*)(smem + kDftWaves * WF);
+  if (nr == 0 && !P.bin_block) {
+    const int nbm = P.nrebin * P.nrebin * P.npix * P.npix;
+    for (int i = threadIdx.x; i < nbm; i += 64 * kDftWaves) s_binmap[i] = P.binmap[i];
+    __syncthreads();
+  }
+  const AwOperand<N, Q, kSplitFp16> aw(nullptr, lane);
+  const int b = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  dft_subap<N, Q, kSplitFp16, false, FULL, NR, false, true>(
+      P, min(b * kDftWaves + wave, P.nvalid - 1), lane, smem + wave * WF, s_binmap, nr, aw, 0u,
+      &Ry);
+}
+
 // Sub-apertures per wave of the same-kind batch kernel (its tiles).
 constexpr int kDftTaskSubaps = 4;
 
@@ -1043,8 +1201,11 @@ static int32_t launch_dft_tasks_n(bool full, int nr, bool noisy, const BatchTask
                                   int ntasks, int total, int grid, size_t lds,
                                   const uint32_t* frame_base, uint32_t frame_off, int remap,
                                   hipStream_t st) {
-  const Frag<PREC>* wtab = wfrag_table<N, Q, PREC>(st);
-  if (!wtab) return fail(SHWFS_ERR_HIP, "DFT batch: building the DFT operand table failed");
+  const Frag<PREC>* wtab = nullptr;
+  if constexpr (PREC != kSplitFp16) {
+    wtab = wfrag_table<N, Q, PREC>(st);
+    if (!wtab) return fail(SHWFS_ERR_HIP, "DFT batch: building the DFT operand table failed");
+  }
   decltype(&sh_dft_tasks_kernel<N, Q, PREC, false, true, 4>) k = nullptr;
 #define SHWFS_PICK(NZ, FL)                                                             \
   switch (nr) {                                                                        \
@@ -1055,7 +1216,9 @@ static int32_t launch_dft_tasks_n(bool full, int nr, bool noisy, const BatchTask
     default: k = sh_dft_tasks_kernel<N, Q, PREC, NZ, FL, 0>; break;                    \
   }
   if (noisy) {
-    if (full) { SHWFS_PICK(true, true) } else { SHWFS_PICK(true, false) }
+    if constexpr (PREC == kSplitFp16)
+      return fail(SHWFS_ERR_ARG, "DFT batch: the split-FP16 stage is noise-free");
+    else if (full) { SHWFS_PICK(true, true) } else { SHWFS_PICK(true, false) }
   } else {
     if (full) { SHWFS_PICK(false, true) } else { SHWFS_PICK(false, false) }
   }
@@ -1099,14 +1262,19 @@ static int32_t launch_dft_t(const ImageParams& p, hipStream_t st, const void* wt
     return fail(SHWFS_ERR_UNSUPPORTED, "DFT spot kernel: LDS footprint exceeds the per-workgroup limit");
   const bool noisy = p.noise > -1.0f;
   const bool full = p.pdiam == L::P16;
-  auto kern = noisy ? (full ? sh_image_dft_kernel<N, Q, PREC, true, true, NR>
-                            : sh_image_dft_kernel<N, Q, PREC, true, false, NR>)
-                    : (full ? sh_image_dft_kernel<N, Q, PREC, false, true, NR>
-                            : sh_image_dft_kernel<N, Q, PREC, false, false, NR>);
-  // the library's cached table, or one the caller has built (wtab_in)
-  const Frag<PREC>* wtab = wtab_in ? static_cast<const Frag<PREC>*>(wtab_in)
-                                   : wfrag_table<N, Q, PREC>(st);
-  if (!wtab) return fail(SHWFS_ERR_HIP, "DFT spot kernel: building the DFT operand table failed");
+  auto kern = full ? sh_image_dft_kernel<N, Q, PREC, false, true, NR>
+                   : sh_image_dft_kernel<N, Q, PREC, false, false, NR>;
+  const Frag<PREC>* wtab = nullptr;
+  if constexpr (PREC == kSplitFp16) {
+    if (noisy) return fail(SHWFS_ERR_ARG, "DFT spot kernel: the split-FP16 stage is noise-free");
+  } else {
+    if (noisy)
+      kern = full ? sh_image_dft_kernel<N, Q, PREC, true, true, NR>
+                  : sh_image_dft_kernel<N, Q, PREC, true, false, NR>;
+    // the library's cached table, or one the caller has built (wtab_in)
+    wtab = wtab_in ? static_cast<const Frag<PREC>*>(wtab_in) : wfrag_table<N, Q, PREC>(st);
+    if (!wtab) return fail(SHWFS_ERR_HIP, "DFT spot kernel: building the DFT operand table failed");
+  }
   if (p.nvalid <= 0) return SHWFS_OK;
   // one wave per sub-aperture, or one workgroup per 64-point sub-aperture;
   // then the workgroups of the fused background
@@ -1130,6 +1298,33 @@ static int32_t launch_dft_n(const ImageParams& p, hipStream_t st, const void* wt
   }
 }
 
+template <int N, int Q, int NR>
+static int32_t launch_dft_ray_t(const ImageParams& p, const RayParams& r, hipStream_t st) {
+  using L = DftLayout<N, Q>;
+  const int nbm = (NR == 0 && !p.bin_block) ? p.nrebin * p.nrebin * p.npix * p.npix : 0;
+  const size_t lds = sizeof(float) * ((size_t)kDftWaves * L::wave_floats(p.npix, NR == 0) + nbm);
+  if (lds > max_lds_per_block())
+    return fail(SHWFS_ERR_UNSUPPORTED, "traced spot kernel: LDS footprint exceeds the per-workgroup limit");
+  auto kern = p.pdiam == L::P16 ? sh_image_dft_ray_kernel<N, Q, true, NR>
+                                : sh_image_dft_ray_kernel<N, Q, false, NR>;
+  const int grid = (p.nvalid + kDftWaves - 1) / kDftWaves;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kDftWaves), lds, st, p, r);
+  SHWFS_LAUNCHED("sh_image_dft_ray_kernel");
+  return SHWFS_OK;
+}
+
+template <int N, int Q>
+static int32_t launch_dft_ray_n(const ImageParams& p, const RayParams& r, hipStream_t st) {
+  switch (dft_register_rebin(p)) {
+    case 4:
+      return dft_half_grid(p, N) ? launch_dft_ray_t<N, Q, 4 | kHalfGrid>(p, r, st)
+                                 : launch_dft_ray_t<N, Q, 4>(p, r, st);
+    case 2: return launch_dft_ray_t<N, Q, 2>(p, r, st);
+    case 1: return launch_dft_ray_t<N, Q, 1>(p, r, st);
+    default: return launch_dft_ray_t<N, Q, 0>(p, r, st);
+  }
+}
+
 // Entry point per operand precision and padded phase side 16*Q; each
 // (PREC, Q) pair is instantiated in a translation unit of its own.  wtab:
 // NULL (the library's table of the shape, built on first use) or a table
@@ -1141,7 +1336,9 @@ int32_t launch_dft_pq(const ImageParams& p, int nfft, hipStream_t st, const void
     switch (nfft) {
       case 16: return launch_dft_n<16, 1, PREC>(p, st, wtab, bg);
       case 32: return launch_dft_n<32, 1, PREC>(p, st, wtab, bg);
-      case 64: return launch_dft_n<64, 1, PREC>(p, st, wtab, bg);
+      case 64:
+        if constexpr (PREC != kSplitFp16) return launch_dft_n<64, 1, PREC>(p, st, wtab, bg);
+        break;
       default: break;
     }
   } else {
@@ -1166,7 +1363,9 @@ int32_t launch_dft_tasks_pq(int nfft, bool full, int nr, bool noisy, const Batch
     switch (nfft) {
       case 16: return launch_dft_tasks_n<16, 1, PREC>(SHWFS_ARGS);
       case 32: return launch_dft_tasks_n<32, 1, PREC>(SHWFS_ARGS);
-      case 64: return launch_dft_tasks_n<64, 1, PREC>(SHWFS_ARGS);
+      case 64:
+        if constexpr (PREC != kSplitFp16) return launch_dft_tasks_n<64, 1, PREC>(SHWFS_ARGS);
+        break;
       default: break;
     }
   } else {
@@ -1232,6 +1431,11 @@ int32_t build_dft_table_pq(int nfft, void* dst, size_t cap, hipStream_t st, size
   return fail(SHWFS_ERR_UNSUPPORTED, "MFMA DFT path: needs nfft in {16, 32, 64} and pdiam <= min(32, nfft)");
 }
 
+extern template int32_t launch_dft_pq<kSplitFp16, 1>(const ImageParams&, int, hipStream_t,
+                                                     const void*, const BgParams&);
+extern template int32_t launch_dft_tasks_pq<kSplitFp16, 1>(
+    int, bool, int, bool, const BatchTask*, const TaskStarts&, const TaskArgs&, int, int, int,
+    size_t, const uint32_t*, uint32_t, int, hipStream_t);
 #define SHWFS_DFT_EXTERN(PREC, Q)                                                         \
   extern template int32_t launch_dft_pq<PREC, Q>(const ImageParams&, int, hipStream_t,  \
                                                  const void*, const BgParams&);         \

@@ -197,6 +197,8 @@ int32_t launch_lgs_kernels(float2* ftlgs, float* lgskern, const float2* prof2d, 
 // shwfs_raytrace.hpp) instead of reading p.phase.
 struct RayParams;
 int32_t launch_image_fft_ray(const ImageParams& p, const RayParams& r, int nfft, hipStream_t s);
+// The split-FP16 kernel with the same (frames of split_fp16_fits).
+int32_t launch_split_ray(const ImageParams& p, const RayParams& r, int nfft, hipStream_t s);
 // The FFT spot kernel with the learned centroider after binning (p.ckind ==
 // SHWFS_CENTROID_MLP): 16 sub-apertures per workgroup, npix 8, nfft 16 or 32.
 int32_t launch_image_fft_mlp(const ImageParams& p, const MlpParams& m, int nfft, hipStream_t s,
@@ -210,6 +212,17 @@ int32_t launch_image_dft_mlp(const ImageParams& p, const MlpParams& m, int nfft,
 // first use) or a table built by build_dft_operand_table.
 int32_t launch_image_dft(const ImageParams& p, int nfft, int method, hipStream_t s,
                          const void* wtab = nullptr, const BgParams& bg = {});
+// Noise-free frames of SHWFS_METHOD_FFT_FP32 on the matrix cores
+// (split-FP16 products of FP32 accuracy, shwfs_image_dft.hpp): whether the
+// frame takes that kernel, and its launch.  Measured a frame, FFT and split:
+// nfft 32, pdiam 16, 80x80 11.4 and 6.5 us, 40x40 8.5 and 5.3; nfft 16, pdiam
+// 8, 74x74 6.7 and 6.0, 8x8 6.1 and 3.4.  The line lies at nfft 32 and windows
+// of 16 points: past it the products lose (pdiam 24, nfft 32: 12.4 and 26.2;
+// nfft 64, pdiam 16, 40x40: 11.8 and 20.2; pdiam 32: 14.4 and 23.2).  A frame
+// that names a workgroup size (wg_size) keeps the in-register FFT, and so does
+// a noisy one: its photon draws would move where a spot's last bit does.
+bool split_fp16_fits(const ImageParams& p, int nfft);
+int32_t launch_image_split(const ImageParams& p, int nfft, hipStream_t s);
 int32_t launch_mfma_probe(const float* A, const float* B, float* D, int method, hipStream_t s);
 // img = sigma * N(0,1) (Philox domain `domain`, element = image index); the
 // call is `call` plus *call_base when call_base is not NULL (device frame

@@ -859,6 +859,9 @@ int32_t SutraWfsSH::comp_generic() {
     clean.noise = -1.0f;
     clean.noise_background = 0.0f;
     clean.d_binimg = d_binimg_notnoisy->get_data();
+    // the noisy launch's own spots (a noise-free FFT frame of the default
+    // workgroup size takes other products, equal to rounding)
+    if (f.noise > -1.0f && clean.wg_size == 0) clean.wg_size = 64;
     shwfs_throw_if(shwfs_sh_comp_image(&g, &clean, stream), "SutraWfsSH::comp_image (roket)");
     const int64_t n = d_bincube->get_nb_elements();
     if (f.noise > -1.0f)

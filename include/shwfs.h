@@ -32,7 +32,10 @@ enum {
 
 /* Computation method of the spot image (shwfs_frame_args.method). */
 enum {
-  SHWFS_METHOD_FFT_FP32 = 0,   /* plain FP32: in-register radix-2 FFT */
+  SHWFS_METHOD_FFT_FP32 = 0,   /* plain FP32: in-register radix-2 FFT; noise-free frames of
+                                  nfft 16 or 32 with windows of up to 16 points and the
+                                  default workgroup size take split-FP16 products of the
+                                  same accuracy on the matrix cores */
   SHWFS_METHOD_DFT_BF16X3 = 1, /* pruned DFT on MFMA, split-BF16x3, FP32 accumulate */
   SHWFS_METHOD_DFT_FP16 = 2    /* pruned DFT on MFMA, FP16 with per-subap scale */
 };
