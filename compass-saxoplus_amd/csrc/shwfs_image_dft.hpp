@@ -402,22 +402,19 @@ __device__ __forceinline__ void field_load(const ImageParams& P, unsigned win, i
   }
 }
 
-// The same phases traced through the layers of R (ray_phase; (i0, j0): the
-// window's corner) instead of read from the rendered screen.
+// The same phases traced through the layers of R ((i0, j0): the window's
+// corner) instead of read from the rendered screen; 0 at points outside a
+// window smaller than the operand tile.
 template <int N, int Q, bool FULL>
-__device__ __forceinline__ void field_trace(const RayParams& R, int i0, int j0, int pdiam_rt,
+__device__ __forceinline__ void field_trace(const RayParams& R, int i0, int j0, int pdiam,
                                             int lane, FieldIn<Q>& f) {
-  constexpr int NP = FieldIn<Q>::NP;
-  const int pdiam = FULL ? DftLayout<N, Q>::P16 : pdiam_rt;
+  static_assert(Q == 1, "field_trace: four points per lane");
+  const int y = lane & 15, x = field_px<Q>(lane, 0);
+  ray_phase4(R, i0 + x, j0 + y, f.ph[0]);
+  if constexpr (!FULL) {
 #pragma unroll
-  for (int ma = 0; ma < Q; ++ma) {
-    const int y = 16 * ma + (lane & 15);
-#pragma unroll
-    for (int j = 0; j < NP; ++j) {
-      const int x = field_px<Q>(lane, j);
-      const bool in = FULL || (x < pdiam && y < pdiam);
-      f.ph[ma][j] = ray_phase(R, i0 + (in ? x : 0), j0 + (in ? y : 0));
-    }
+    for (int j = 0; j < 4; ++j)
+      if (x + j >= pdiam || y >= pdiam) f.ph[0][j] = 0.0f;
   }
 }
 
@@ -1141,7 +1138,7 @@ void sh_image_dft_kernel(ImageParams P, const Frag<PREC>* wtab, BgParams bg) {
 // The split-FP16 spot kernel with the guide-star raytrace in its field stage
 // (noise-free): the npup^2 screen is neither written nor read back.
 template <int N, int Q, bool FULL, int NR>
-__global__ __launch_bounds__(64 * kDftWaves)
+__global__ __launch_bounds__(64 * kDftWaves) __attribute__((amdgpu_waves_per_eu(4)))
 void sh_image_dft_ray_kernel(ImageParams P, RayParams Ry) {
   constexpr int nr = NR & 7;
   using L = DftLayout<N, Q>;

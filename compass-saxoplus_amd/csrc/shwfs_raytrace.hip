@@ -33,6 +33,7 @@ int32_t ray_params(const shwfs_layer* layers, int32_t nlayers, int32_t nx, int32
     l.delta = a.delta;
     l.dx = a.dx;
     l.dy = a.dy;
+    l.axis = l.c == 1.0f && l.s == 0.0f;
   }
   *out = r;
   return SHWFS_OK;
