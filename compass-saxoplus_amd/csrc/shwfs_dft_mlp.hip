@@ -25,7 +25,8 @@ constexpr int kDmN = 32, kDmNrc = 4 | kHalfGrid;
 template <int PREC, bool NOISE>
 __global__ __launch_bounds__(kDmThreads) void sh_image_dft_mlp_kernel(ImageParams P, MlpParams M,
                                                                       const Frag<PREC>* wtab,
-                                                                      BgParams bg, int slot) {
+                                                                      BgParams bg, int slot,
+                                                                      int wpos) {
   if constexpr (NOISE) {
     if ((int)blockIdx.x >= bg.spot_blocks) {
       draw_background<kDmThreads>(P, bg, (int)blockIdx.x - bg.spot_blocks);
@@ -36,13 +37,18 @@ __global__ __launch_bounds__(kDmThreads) void sh_image_dft_mlp_kernel(ImageParam
   const int tid = (int)threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s0 = xcd_remap(blockIdx.x, bg.spot_blocks) * kDmWaves;
+  // the network's parameters, on their way while the spots are computed (read
+  // layer by layer from global memory they cost 1.8 of a 40x40 frame's 17.0 us)
+  mlp::LdsWeights<kDmThreads> W(reinterpret_cast<char*>(smem + wpos));
+  W.fetch(M.params, tid);
   {
     // spare waves of the last workgroup recompute the last sub-aperture (the
     // same values to the same addresses); their rows are not used
     const AwOperand<kDmN, 1, PREC> aw(wtab, lane);
-    dft_subap<kDmN, 1, PREC, NOISE, true, kDmNrc, true>(P, min(s0 + wave, P.nvalid - 1), lane,
-                                                       smem + wave * slot, P.binmap, kDmNrc & 7,
-                                                       aw);
+    auto mid = [&] { W.store(tid); };
+    dft_subap<kDmN, 1, PREC, NOISE, true, kDmNrc, true, false>(
+        P, min(s0 + wave, P.nvalid - 1), lane, smem + wave * slot, P.binmap, kDmNrc & 7, aw, 0u,
+        nullptr, mid);
   }
   __syncthreads();
   // the spots (wave w's at the start of its slot) into registers, then, past
@@ -65,8 +71,7 @@ __global__ __launch_bounds__(kDmThreads) void sh_image_dft_mlp_kernel(ImageParam
     T.x[k * mlp::SX + c] = (__bf16)(v[e] * M.xs);
   }
   // starts with a barrier
-  mlp::tile_forward<kDmTile>(M.params, mlp::Fp32Weights{M.params}, T,
-                                                      tid);
+  mlp::tile_forward<kDmTile>(W, T, tid);
   for (int k = wave; k < rows; k += kDmWaves)
     mlp::spot_slopes(spots[k * 64 + lane], lane, s0 + k, P.nvalid, T.y[k * mlp::NOUT],
                      T.y[k * mlp::NOUT + 1], M.lo, M.hi, P.coffset, P.cscale, M.ys, P.ref,
@@ -83,7 +88,8 @@ int32_t launch_dft_mlp_p(const ImageParams& p, const MlpParams& m, hipStream_t s
   size_t floats = (size_t)kDmWaves * slot;
   const size_t mlp_floats = (size_t)kDmTile * 64 + mlp::Lds<kDmTile>::bytes() / sizeof(float);
   if (floats < mlp_floats) floats = mlp_floats;
-  const size_t lds = floats * sizeof(float);
+  const int wpos = (int)((floats + 3) & ~(size_t)3);  // the parameters, 16-byte aligned
+  const size_t lds = wpos * sizeof(float) + mlp::LdsWeights<kDmThreads>::bytes();
   if (lds > max_lds_per_block())
     return fail(SHWFS_ERR_UNSUPPORTED, "DFT + MLP kernel: LDS footprint exceeds the per-workgroup limit");
   bg.spot_blocks = (p.nvalid + kDmWaves - 1) / kDmWaves;
@@ -91,10 +97,10 @@ int32_t launch_dft_mlp_p(const ImageParams& p, const MlpParams& m, hipStream_t s
   const int grid = bg.spot_blocks + (noisy ? (bg.n + kDmThreads - 1) / kDmThreads : 0);
   if (noisy)
     hipLaunchKernelGGL((sh_image_dft_mlp_kernel<PREC, true>), dim3(grid), dim3(kDmThreads), lds,
-                       st, p, m, wtab, bg, slot);
+                       st, p, m, wtab, bg, slot, wpos);
   else
     hipLaunchKernelGGL((sh_image_dft_mlp_kernel<PREC, false>), dim3(grid), dim3(kDmThreads), lds,
-                       st, p, m, wtab, bg, slot);
+                       st, p, m, wtab, bg, slot, wpos);
   SHWFS_LAUNCHED("sh_image_dft_mlp_kernel");
   return SHWFS_OK;
 }

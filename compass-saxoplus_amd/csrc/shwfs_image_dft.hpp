@@ -917,13 +917,18 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
 // (nr == 0), the moment totals use the 192 doubles after the spot (nr > 0)
 // or at the start, over the dead |F|^2 image (nr == 0).  KEEP: no centroider;
 // the spot-cube values stay in the spot.
-// RAY: the window's phases are traced through the layers of *ray.
+// RAY: the window's phases are traced through the layers of *ray.  mid: called
+// between the spot and its tail.
+struct NoMid {
+  __device__ __forceinline__ void operator()() const {}
+};
 template <int N, int Q, int PREC, bool NOISE, bool FULL, int NRC = -1, bool KEEP = false,
-          bool RAY = false>
+          bool RAY = false, class Mid = NoMid>
 __device__ __forceinline__ void dft_subap(const ImageParams& P, const int s, const int lane,
                                           float* smem, const int* bm, const int nr_rt,
                                           const AwOperand<N, Q, PREC>& aw,
-                                          unsigned call_add = 0u, const RayParams* ray = nullptr) {
+                                          unsigned call_add = 0u, const RayParams* ray = nullptr,
+                                          const Mid& mid = Mid()) {
   using L = DftLayout<N, Q>;
   const int nr = NRC >= 0 ? (NRC & 7) : nr_rt;
   SubapScalars pre;
@@ -945,6 +950,7 @@ __device__ __forceinline__ void dft_subap(const ImageParams& P, const int s, con
   dft_spot<N, Q, PREC, FULL, NRC>(P, lane, smem, bin, bm, nr_rt, aw, fin, of, win, unit,
                                   inten_scale);
   wave_lds_sync();
+  mid();
   const float I = spot_sum<64>(bin, npix * npix, true, lane);
   void* red = nr > 0 ? smem + spot_f : smem;
   finish_spot<64, NOISE, KEEP>(P, s, true, lane, bin, I, inten_scale, call_add, red, &pre);

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kMlpThreads) void sh_image_fft_mlp_kernel(ImagePara
   for (int i = S * 64 + tid; i < kMlpTile * 64; i += TPB)
     T.x[(i >> 6) * mlp::SX + (i & 63)] = (__bf16)0.0f;
   // starts with a barrier
-  mlp::tile_forward<kMlpTile>(M.params, mlp::Fp32Weights{M.params}, T, tid);
+  mlp::tile_forward<kMlpTile>(mlp::Fp32Weights{M.params}, T, tid);
   const int lane = tid & 63, w = tid >> 6;
   for (int k = w; k < rows; k += NW)
     mlp::spot_slopes(spots[k * 64 + lane], lane, s0 + k, P.nvalid, T.y[k * mlp::NOUT],

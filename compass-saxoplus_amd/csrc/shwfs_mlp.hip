@@ -59,7 +59,7 @@ __global__ __launch_bounds__(TPB) void mlp_tile_kernel(const float* __restrict__
   const int rows = (int)((n - row0) < TS ? (n - row0) : TS);
   const int tid = threadIdx.x;
   load_rows(x, row0, rows, x_scale, L);
-  mlp::tile_forward<TS>(P, Bf16Weights{W1b, W2b}, L, tid);
+  mlp::tile_forward<TS>(Bf16Weights{P, W1b, W2b}, L, tid);
   if (tid < rows * NOUT) y[(row0 + tid / NOUT) * NOUT + tid % NOUT] = L.y[tid];
 }
 
@@ -508,7 +508,7 @@ __global__ __launch_bounds__(TPB) void mlp_centroid_kernel(
     const int sl = i / NIN, c = i % NIN;
     L.x[sl * SX + c] = (__bf16)(sl < rows ? pixel(row0 + sl, c) * x_scale : 0.0f);
   }
-  mlp::tile_forward<TS>(P, Bf16Weights{W1b, W2b}, L, (int)threadIdx.x);
+  mlp::tile_forward<TS>(Bf16Weights{P, W1b, W2b}, L, (int)threadIdx.x);
   // flux and CoG from the raw pixels: one wave per 8 sub-apertures
   for (int k = 0; k < TS / 4; ++k) {
     const int sl = w * (TS / 4) + k;

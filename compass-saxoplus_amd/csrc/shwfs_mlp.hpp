@@ -56,8 +56,10 @@ __device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cas
 // Weight operands from bf16 copies of W1 and W2 (the training and
 // stand-alone inference kernels, which convert them once per launch).
 struct Bf16Weights {
+  const float* P;
   const __bf16* W1b;
   const __bf16* W2b;
+  __device__ float par(int i) const { return P[i]; }
   __device__ bf16x8 w1(int row, int k) const { return ld8(W1b + row * NIN + k); }
   __device__ bf16x8 w2(int row, int k) const { return ld8(W2b + row * NH + k); }
 };
@@ -76,6 +78,69 @@ struct Fp32Weights {
   }
   __device__ bf16x8 w1(int row, int k) const { return cvt8(P + OW1 + row * NIN + k); }
   __device__ bf16x8 w2(int row, int k) const { return cvt8(P + OW2 + row * NH + k); }
+  __device__ float par(int i) const { return P[i]; }
+};
+
+// The same operands and parameters from LDS: fetched into registers by the
+// workgroup's THREADS threads when it starts (fetch), converted and stored
+// once they have arrived (store), so that the network's three layers wait for
+// no global memory.
+template <int THREADS>
+struct LdsWeights {
+  static constexpr int S1 = NIN + 8, S2 = NH + 8;  // row strides, 16-byte rows
+  static constexpr int NSMALL = 2 * NH + NOUT * NH + NOUT;  // b1, b2, W3, b3
+  static constexpr int Q1 = NH * NIN / 4 / THREADS, Q2 = NH * NH / 4 / THREADS;
+  static_assert(Q1 * THREADS * 4 == NH * NIN && Q2 * THREADS * 4 == NH * NH && NSMALL <= 2 * THREADS,
+                "LdsWeights: whole float4 per thread");
+  __bf16* W1s;
+  __bf16* W2s;
+  float* small;
+  float4 r1[Q1], r2[Q2];
+  float rs[2];
+  static constexpr size_t bytes() {
+    return sizeof(__bf16) * (size_t)NH * (S1 + S2) + sizeof(float) * (size_t)((NSMALL + 3) & ~3);
+  }
+  __device__ explicit LdsWeights(char* base) {
+    W1s = reinterpret_cast<__bf16*>(base);
+    W2s = W1s + NH * S1;
+    small = reinterpret_cast<float*>(W2s + NH * S2);
+  }
+  // parameter index of small value i
+  __device__ static int small_param(int i) { return i < NH ? OB1 + i : OB2 + (i - NH); }
+  __device__ void fetch(const float* P, int tid) {
+    static_assert(OW3 == OB2 + NH && OB3 == OW3 + NOUT * NH, "b2, W3 and b3 are consecutive");
+#pragma unroll
+    for (int q = 0; q < Q1; ++q) r1[q] = reinterpret_cast<const float4*>(P + OW1)[tid + q * THREADS];
+#pragma unroll
+    for (int q = 0; q < Q2; ++q) r2[q] = reinterpret_cast<const float4*>(P + OW2)[tid + q * THREADS];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = tid + q * THREADS;
+      rs[q] = P[small_param(i < NSMALL ? i : 0)];
+    }
+  }
+  __device__ static void put4(__bf16* d, const float4& v) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<bf16x4*>(d) = bf16x4{(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+  }
+  __device__ void store(int tid) const {
+#pragma unroll
+    for (int q = 0; q < Q1; ++q) {
+      const int i = 4 * (tid + q * THREADS);
+      put4(W1s + (i / NIN) * S1 + i % NIN, r1[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < Q2; ++q) {
+      const int i = 4 * (tid + q * THREADS);
+      put4(W2s + (i / NH) * S2 + i % NH, r2[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (tid + q * THREADS < NSMALL) small[tid + q * THREADS] = rs[q];
+  }
+  __device__ bf16x8 w1(int row, int k) const { return ld8(W1s + row * S1 + k); }
+  __device__ bf16x8 w2(int row, int k) const { return ld8(W2s + row * S2 + k); }
+  __device__ float par(int i) const { return small[i < OB2 ? i - OB1 : i - OB2 + NH]; }
 };
 
 // Forward of the TS samples in L.x (bf16, scaled inputs) into LDS (z1, h1,
@@ -86,8 +151,7 @@ struct Fp32Weights {
 // tile.  tid: the thread index.
 // g2 receives gelu(z2) in fp32, which the last layer reads.
 template <int TS, class WS>
-__device__ __forceinline__ void tile_forward(const float* __restrict__ P, const WS& ws,
-                                             const Lds<TS>& L, int tid) {
+__device__ __forceinline__ void tile_forward(const WS& ws, const Lds<TS>& L, int tid) {
   const int lane = tid & 63, w = tid >> 6;
   __syncthreads();
   if (w < 4) {
@@ -108,7 +172,7 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * mi + 4 * (lane >> 4) + v;
-          const float z = acc[v] + P[OB1 + col];
+          const float z = acc[v] + ws.par(OB1 + col);
           L.h1[row * SH + col] = (__bf16)gelu(z);
         }
       }
@@ -132,7 +196,7 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * mi + 4 * (lane >> 4) + v;
-          const float z = acc[v] + P[OB2 + col];
+          const float z = acc[v] + ws.par(OB2 + col);
           const float g = gelu(z);
           L.g2[row * SZ + col] = g;
         }
@@ -154,11 +218,11 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ P, const 
 #pragma unroll 4
     for (int j = 0; j < NH / PARTS; ++j) {
       const int k = part + PARTS * j;
-      acc += L.g2[s * SZ + k] * P[OW3 + o * NH + k];
+      acc += L.g2[s * SZ + k] * ws.par(OW3 + o * NH + k);
     }
 #pragma unroll
     for (int m = 1; m < PARTS; m <<= 1) acc += __shfl_xor(acc, m, PARTS);
-    if (part == 0) L.y[s * NOUT + o] = acc + P[OB3 + o];
+    if (part == 0) L.y[s * NOUT + o] = acc + ws.par(OB3 + o);
   }
   __syncthreads();
 }
