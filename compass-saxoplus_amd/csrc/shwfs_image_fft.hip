@@ -26,6 +26,54 @@ __global__ __launch_bounds__(TPB) void sh_image_fft_kernel(ImageParams P, BgPara
   fft_tile<N, R, TPB, NOISE>(P, xcd_remap(blockIdx.x, bg.spot_blocks) * S, smem, s_binmap);
 }
 
+// Noisy frames, one sub-aperture per wave (fft_wave), kFftNoisyWaves waves per
+// workgroup; workgroups past bg.spot_blocks draw the fused background.
+constexpr int kFftNoisyWaves = 4;
+// Up to two such waves per SIMD (1,024 of them): the samplers' serial chain
+// sets the time, and a lane draws one pixel instead of 64 / N in turn.  Past
+// that the lanes that idle in the transforms cost as much.  Per frame, N lanes
+// and a wave per sub-aperture: nfft 32, 8x8 px, 40x40 (1,256) 20.4 and 15.5
+// us, 50x50 (1,944) 20.9 and 16.1, 60x60 (2,792) 23.3 and 23.8, 80x80 35.5 and
+// 34.3; nfft 16, 40x40 24.3 and 13.7, 74x74 (4,268) 24.6 and 28.7.  (nfft 64
+// has 64 lanes already.)
+constexpr int kFftNoisyMax = 2048;
+template <int N, int R>
+__global__ __launch_bounds__(64 * kFftNoisyWaves) __attribute__((amdgpu_waves_per_eu(2)))
+void sh_image_fft_noisy_kernel(ImageParams P, BgParams bg) {
+  using L = FftLayout<N, R>;
+  if ((int)blockIdx.x >= bg.spot_blocks) {
+    draw_background<64 * kFftNoisyWaves>(P, bg, (int)blockIdx.x - bg.spot_blocks);
+    return;
+  }
+  extern __shared__ float smem[];
+  const int slot = L::slot_floats(P.pdiam, P.npix);
+  int* s_binmap = (int*)(smem + kFftNoisyWaves * slot);
+  if (!P.bin_block) {
+    const int nbm = P.nrebin * P.nrebin * P.npix * P.npix;
+    for (int i = threadIdx.x; i < nbm; i += 64 * kFftNoisyWaves) s_binmap[i] = P.binmap[i];
+    __syncthreads();
+  }
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // spare waves of the last workgroup recompute the last sub-aperture
+  const int s = min(xcd_remap(blockIdx.x, bg.spot_blocks) * kFftNoisyWaves + wave, P.nvalid - 1);
+  fft_wave<N, R>(P, s, (int)threadIdx.x & 63, smem + wave * slot, s_binmap);
+}
+
+template <int N, int R>
+static int32_t launch_fft_noisy(const ImageParams& p, hipStream_t st, BgParams bg) {
+  using L = FftLayout<N, R>;
+  constexpr int TPB = 64 * kFftNoisyWaves;
+  const int nbm = p.bin_block ? 0 : p.nrebin * p.nrebin * p.npix * p.npix;
+  const size_t lds = sizeof(float) * ((size_t)kFftNoisyWaves * L::slot_floats(p.pdiam, p.npix) + nbm);
+  if (lds > max_lds_per_block())
+    return fail(SHWFS_ERR_UNSUPPORTED, "spot kernel: LDS footprint exceeds the per-workgroup limit");
+  bg.spot_blocks = (p.nvalid + kFftNoisyWaves - 1) / kFftNoisyWaves;
+  hipLaunchKernelGGL((sh_image_fft_noisy_kernel<N, R>), dim3(bg.spot_blocks + (bg.n + TPB - 1) / TPB),
+                     dim3(TPB), lds, st, p, bg);
+  SHWFS_LAUNCHED("sh_image_fft_noisy_kernel");
+  return SHWFS_OK;
+}
+
 template <int N, int R, int TPB>
 static int32_t launch_fft_nrt(const ImageParams& p, hipStream_t st, BgParams bg) {
   using L = FftLayout<N, R>;
@@ -49,6 +97,11 @@ template <int N, int R>
 static int32_t launch_fft_nr(const ImageParams& p, hipStream_t st, const BgParams& bg) {
   // workgroup size: 64 lanes by default (more, smaller workgroups spread the
   // sub-apertures evenly over the 256 CUs); 256 on request (tuning)
+  // noisy frames of few sub-apertures: one wave each (kFftNoisyMax)
+  if constexpr (N == 16 || N == 32) {
+    if (p.tpb == 0 && p.noise > -1.0f && p.nvalid <= kFftNoisyMax)
+      return launch_fft_noisy<N, R>(p, st, bg);
+  }
   if (p.tpb == 256) return launch_fft_nrt<N, R, 256>(p, st, bg);
   if (p.tpb == 128 && N <= 128) return launch_fft_nrt<N, R, 128>(p, st, bg);
   return launch_fft_nrt<N, R, 64>(p, st, bg);

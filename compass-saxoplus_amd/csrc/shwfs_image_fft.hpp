@@ -140,4 +140,81 @@ __device__ __forceinline__ void fft_tile(const ImageParams& P, int s0, float* sm
   tile_sync<TPB>();
 }
 
+// Sub-aperture s (< nvalid) by one whole wave (noisy frames of few
+// sub-apertures): the spot of fft_tile, bit for bit (the same transforms by N
+// lanes in the same order, the flux summed as N lanes sum it), since a spot's
+// last bit can move a photon count; then one noisy pixel per lane of an 8x8
+// spot where N lanes draw 64 / N in turn.  smem: the wave's slot (slot_floats).
+template <int N, int R>
+__device__ __forceinline__ void fft_wave(const ImageParams& P, int s, int lane, float* smem,
+                                         const int* bm) {
+  using L = FftLayout<N, R>;
+  constexpr int M = L::M, PS = L::PS;
+  const int pdiam = P.pdiam, PE = L::pe(pdiam), npix2 = P.npix * P.npix;
+  float2* E = (float2*)smem;
+  float2* G = (float2*)smem;  // aliases E, then hr aliases G
+  float* hr = smem;
+  float* bin = smem + (L::slot_floats(pdiam, P.npix) - ((npix2 + 3) & ~3));
+  SubapScalars pre;
+  pre.load(P, s);
+  load_fields<64, (M * M + 63) / 64, false>(P, s, true, lane, (float*)E, PE, 0);
+  wave_lds_sync();
+  {  // rows
+    float re[M], im[M];
+    const int y = lane / R, r = lane % R;
+    const bool on = y < pdiam;  // lane < N R M / N = M R
+#pragma unroll
+    for (int x = 0; x < M; ++x) {
+      float2 v = make_float2(0.f, 0.f);
+      if (on && x < pdiam) v = E[y * PE + x];
+      re[x] = v.x;
+      im[x] = v.y;
+    }
+    if constexpr (R == 2) {
+      if (r) PreTw<N, M, 0>::run(re, im);
+    }
+    fft_reg<M>(re, im);
+    wave_lds_sync();
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < M; ++k) G[(R * k + r) * PS + y] = make_float2(re[k], im[k]);
+    }
+  }
+  wave_lds_sync();
+  {  // columns
+    float gr[M], gi[M];
+    const bool on = lane < N;
+#pragma unroll
+    for (int y = 0; y < M; ++y) {
+      float2 v = make_float2(0.f, 0.f);
+      if (on && y < pdiam) v = G[lane * PS + y];
+      gr[y] = v.x;
+      gi[y] = v.y;
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+      float zr[M], zi[M];
+#pragma unroll
+      for (int y = 0; y < M; ++y) {
+        zr[y] = gr[y];
+        zi[y] = gi[y];
+      }
+      if (rr == 1) PreTw<N, M, 0>::run(zr, zi);
+      fft_reg<M>(zr, zi);
+      if (on) {
+#pragma unroll
+        for (int k = 0; k < M; ++k) hr[lane + (R * k + rr) * N] = zr[k] * zr[k] + zi[k] * zi[k];
+      }
+    }
+  }
+  wave_lds_sync();
+  (void)bin_gather<64, N>(P, true, lane, hr, bin, bm);
+  wave_lds_sync();
+  float part = 0.0f;  // fft_tile's sums: N lanes, pixels p, p + N, ... in turn
+  for (int p = lane % N; p < npix2; p += N) part += bin[p];
+  const float I = lane_group_sum<N>(part);
+  finish_spot<64, true>(P, s, true, lane, bin, I, 1.0f, 0u, nullptr, &pre);
+}
+
 }  // namespace shwfs
