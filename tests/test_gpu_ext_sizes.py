@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("nx,pd,nfft,nrebin,npix,conv", [
     (1, 8, 16, 2, 8, True), (2, 16, 16, 2, 7, True), (3, 5, 16, 3, 8, False),
-    (2, 8, 16, 3, 8, True), (2, 12, 16, 4, 16, False), (4, 7, 16, 4, 16, True),
-    (3, 16, 32, 4, 8, True), (5, 32, 32, 2, 10, True), (2, 20, 32, 4, 16, False),
+    (2, 8, 16, 3, 8, True), (2, 12, 16, 4, 15, False), (4, 7, 16, 4, 15, True),
+    (3, 16, 32, 4, 8, True), (5, 32, 32, 2, 10, True), (2, 20, 32, 4, 15, False),
     (3, 13, 32, 3, 13, True), (2, 40, 64, 4, 16, True), (3, 64, 64, 3, 9, True)])
 def test_frame_matches_oracle(nx, pd, nfft, nrebin, npix, conv):
     c = configs.sh_config(0.3 * nx, nx + (nx * pd) % 2, pd, npix, nfft, nrebin, cobs=0.0,
