@@ -111,6 +111,7 @@ int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, hipStream
     *lds = sizeof(float) * (size_t)t.per_tile * slot;
   } else {
     const int prec = products ? kSplitFp16 : tile.method;
+    if (products) t.P.fp64 = 1;  // as those frames alone
     if (!dft_kind(nfft, pdiam, prec, &t.kind))
       return fail(SHWFS_ERR_UNSUPPORTED, "batch: DFT stage needs nfft in {16, 32, 64}, pdiam <= 32");
     t.per_tile = kDftTaskSubaps;

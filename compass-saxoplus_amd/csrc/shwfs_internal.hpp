@@ -200,7 +200,7 @@ int32_t launch_image_fft_ray(const ImageParams& p, const RayParams& r, int nfft,
 // The split-FP16 kernel with the same (frames of split_fp16_fits).
 int32_t launch_split_ray(const ImageParams& p, const RayParams& r, int nfft, hipStream_t s);
 // The FFT spot kernel with the learned centroider after binning (p.ckind ==
-// SHWFS_CENTROID_MLP): 16 sub-apertures per workgroup, npix 8, nfft 16 or 32.
+// SHWFS_CENTROID_MLP): 256 / nfft sub-apertures per workgroup, npix 8, nfft 16 or 32.
 int32_t launch_image_fft_mlp(const ImageParams& p, const MlpParams& m, int nfft, hipStream_t s,
                              const BgParams& bg = {});
 // The same after MFMA DFT spots (shwfs_dft_mlp.hip) for the shapes

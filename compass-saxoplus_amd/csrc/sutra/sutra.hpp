@@ -263,7 +263,7 @@ class SutraWfsSH : public SutraWfs {
   CarmaObj<int32_t>* d_validpuppixx;
   CarmaObj<int32_t>* d_validpuppixy;
   // field stop (set_field_stop): d_fsamplipup is the n x npup work array of
-  // the transforms; the spot kernels read the stopped field as the amplitude
+  // the transforms (scratch, in the kernels' tiled order); the spot kernels read the stopped field as the amplitude
   // d_fsampl and the phase d_fsphase ([npup^2] each).  d_fsamplifoc stays
   // NULL: the focal-plane field is never stored whole.
   CarmaObj<hipFloatComplex>* d_fsamplipup;
@@ -305,7 +305,8 @@ class SutraWfsSH : public SutraWfs {
   int32_t set_bincube(float* bincube, int32_t nElem);
   int32_t set_field_stop(PlanMap& campli_plans, float* field_stop, int32_t N);
 
-  // Spot computation method (SHWFS_METHOD_*); FP32 FFT by default.
+  // Spot computation method (SHWFS_METHOD_*); the FFT method by default, whose
+  // noise-free frames take the split-FP16 products unless a wg_size is set.
   int32_t set_method(int32_t method);
   int32_t get_method() const { return campli_plan ? campli_plan->method : SHWFS_METHOD_FFT_FP32; }
   int32_t set_wg_size(int32_t wg_size);

@@ -419,8 +419,10 @@ int32_t shwfs_upload(void* d_dst, int64_t dst_elems, const void* h_src, int64_t 
 typedef struct shwfs_batch shwfs_batch; /* opaque */
 typedef struct shwfs_batch_tile {
   int32_t method; /* SHWFS_METHOD_* used for this WFS in the batch */
-  int32_t split;  /* FFT stage: 1, or 2 (row transforms split in two, needs
-                     2*nphase <= nfft); 0 = 2 when allowed.  Ignored by DFT. */
+  int32_t split;  /* FFT method: 1, or 2 (row transforms split in two, needs
+                     2*nphase <= nfft); 0 = the split-FP16 products where a
+                     noise-free batch allows them (as SHWFS_METHOD_FFT_FP32),
+                     else 2 when allowed.  Ignored by DFT. */
 } shwfs_batch_tile;
 /* frames[i].method is the initial method of WFS i (wg_size is ignored).
  * Refused (SHWFS_ERR_UNSUPPORTED): ntot != nfft, kernconv, LGS kernels, layers, and the
@@ -460,7 +462,8 @@ int32_t shwfs_batch_autotune(shwfs_batch* batch, uint32_t method_mask, int32_t r
  * matrix cores, FP32 accumulation, FP32 master parameters.
  * d_params: flat [SHWFS_MLP_NPARAM] = W1 (128x64 row-major), b1 (128),
  * W2 (128x128), b2 (128), W3 (2x128), b3 (2).  d_work: shwfs_mlp_work_bytes()
- * of device scratch for the bf16 weight copies.  Inputs x: [n][64] spots
+ * of device scratch for the bf16 weight copies and shwfs_mlp_loss_grad's
+ * partial gradients (one call at a time uses it).  Inputs x: [n][64] spots
  * (pixel px + 8*py), multiplied by x_scale; outputs / targets [n][2] in
  * pixels.  Loss: mean over samples and outputs of (y - t)^2. */
 #define SHWFS_MLP_NPARAM 25090
