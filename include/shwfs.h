@@ -116,7 +116,8 @@ typedef struct shwfs_centroid_args {
   float* d_slopes;         /* [2*nvalid] */
   float* d_intensities;    /* [nvalid] centroider flux */
   int32_t slope_order;     /* 0 untied (x..., y...), 1 interlaced (x, y, x, y...) */
-  int32_t fp64_moments;    /* 1: flux and first moments summed in float64 */
+  int32_t fp64_moments;    /* 1: flux and first moments summed in float64 (frames
+                               on the split-FP16 products always sum them so) */
   /* SHWFS_CENTROID_MLP only (fused into the spot kernel: the FFT method with
    * 8x8-pixel spots at nfft 16 or 32, or an MFMA method at nfft 32 with
    * 16-point windows and 8x8 pixels binned 4x4 about the grid centre): as
