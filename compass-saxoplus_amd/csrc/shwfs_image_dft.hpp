@@ -588,9 +588,22 @@ __device__ __forceinline__ void spot_bin_block(const f32x4 (&fb)[DftLayout<N, Q>
   }
 }
 
+// Exponent of G of a scaled field: the bound amax = pdiam * max |E| goes to
+// [2^14, 2^15); 2^t is the table's, the rest the field's.  Bounds below
+// 2^(-113 - t) take the largest field factor a float holds, 2^127; a zero or
+// subnormal bound the table's scale alone.
+__device__ __forceinline__ int field_exponent(float amax, int t) {
+  const int ex = ((__float_as_int(amax) >> 23) & 0xff) - 127;  // ilogb for normal amax
+  return amax >= 1.17549435e-38f ? min(14 - ex, t + 127) : t;
+}
+// 2^(e - t), the factor on the field
+__device__ __forceinline__ float field_factor(int e, int t) {
+  return __int_as_float((127 + e - t) << 23);  // -125 <= e - t <= 127
+}
+
 // Binned spot of sub-aperture s (< nvalid, uniform over the wave), before
 // the flux normalisation, into bin (npix^2 floats of LDS, x fastest), in units
-// of 1/inten_scale (returned through inten_scale).  hr: N^2 floats of LDS for
+// of 2^-inten_exp (returned through inten_exp).  hr: N^2 floats of LDS for
 // the |F|^2 image (nr == 0 only); bm: the binmap table (LDS or global) used
 // when nr == 0; nr: register rebin factor (dft_register_rebin), fixed at
 // compile time by NRC >= 0 (NRC & 7; bit kHalfGrid: the half-grid 4x4 form,
@@ -605,7 +618,7 @@ __device__ __forceinline__ void dft_spot(const ImageParams& P, const int lane, f
                                          float* bin, const int* bm, const int nr_rt,
                                          const AwOperand<N, Q, PREC>& aw, const FieldIn<Q>& fin,
                                          const float (&of)[Q][FieldIn<Q>::NP], const unsigned win,
-                                         const bool unit, float& inten_scale, const int part = 0) {
+                                         const bool unit, int& inten_exp, const int part = 0) {
   static_assert(PARTS == 1 || (NRC >= 0 && (NRC & 7) > 0 && (N / 16) % PARTS == 0),
                 "dft_spot: a shared sub-aperture needs register binning and whole kx blocks");
   const int nr = NRC >= 0 ? (NRC & 7) : nr_rt;
@@ -637,10 +650,8 @@ __device__ __forceinline__ void dft_spot(const ImageParams& P, const int lane, f
 #pragma unroll
             for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(ev[ma][ks][e]));
         const float amax = wave_max(m) * (float)pdiam;
-        const int ex = ((__float_as_int(amax) >> 23) & 0xff) - 127;  // ilogb for normal amax
-        // zero or subnormal bound: the table's scale alone
-        e_total = amax >= 1.17549435e-38f ? 14 - ex : t;
-        const float fscale = __int_as_float((127 + e_total - t) << 23);  // |e_total - t| < 127
+        e_total = field_exponent(amax, t);
+        const float fscale = field_factor(e_total, t);
 #pragma unroll
         for (int ma = 0; ma < Q; ++ma)
 #pragma unroll
@@ -685,8 +696,8 @@ __device__ __forceinline__ void dft_spot(const ImageParams& P, const int lane, f
         }
   }
   // F carries 2^(e_total + t) (stage B's table scale too): |F|^2 is scaled
-  // back by 2^(-2 (e_total + t)) (may be subnormal)
-  inten_scale = ldexpf(1.0f, -2 * (e_total + t));
+  // back by 2^(-2 (e_total + t)), past a float's own range for faint windows
+  inten_exp = -2 * (e_total + t);
 
   // ---- stage B per kx tile: F = A_W [Gr ; Gi]; K step ks takes the Gr and
   // Gi tiles of the kx block (Q == 1), or the two row blocks of Gr (ks = 0)
@@ -847,7 +858,7 @@ __device__ __forceinline__ float pair_half_max(float m) {
 }
 
 // The binned spots of sub-apertures a and b (see above) into bin_a, bin_b,
-// in units of 1 / scale_a and 1 / scale_b.
+// in units of 2^-exp_a and 2^-exp_b.
 template <int N, int PREC, int NRC>
 __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int lane, float* bin_a,
                                               float* bin_b, const AwOperand<N, 1, PREC>& aw,
@@ -855,7 +866,7 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
                                               const float (&of)[1][FieldIn<1>::NP],
                                               const unsigned win_a, const unsigned win_b,
                                               const bool unit_a, const bool unit_b,
-                                              float& scale_a, float& scale_b) {
+                                              int& exp_a, int& exp_b) {
   using L = DftLayout<N, 1>;
   using F = Frag<PREC>;
   static_assert(L::MT == 2 && L::KS == 1 && L::NTB == 1, "dft_spot_pair: the 16-point stage");
@@ -874,10 +885,9 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
 #pragma unroll
       for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(ev[0][0][e]));
       const float amax = pair_half_max(m) * (float)P.pdiam;
-      const int ex = ((__float_as_int(amax) >> 23) & 0xff) - 127;  // ilogb for normal amax
       const bool unit = (lane & 8) ? unit_b : unit_a;
-      const int e_lane = unit ? t : (amax >= 1.17549435e-38f ? 14 - ex : t);
-      const float fscale = __int_as_float((127 + e_lane - t) << 23);  // |e_lane - t| < 127
+      const int e_lane = unit ? t : field_exponent(amax, t);
+      const float fscale = field_factor(e_lane, t);
 #pragma unroll
       for (int e = 0; e < 8; ++e) ev[0][0][e] *= fscale;
       e_a = __builtin_amdgcn_readlane(e_lane, 0);  // lane 0: half a
@@ -892,8 +902,8 @@ __device__ __forceinline__ void dft_spot_pair(const ImageParams& P, const int la
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     ga[nt] = mma(ae, aw.get(nt, 0), acc);
   }
-  scale_a = ldexpf(1.0f, -2 * (e_a + t));
-  scale_b = ldexpf(1.0f, -2 * (e_b + t));
+  exp_a = -2 * (e_a + t);
+  exp_b = -2 * (e_b + t);
   const int o = P.bin_origin, npix = P.npix;
   const int nr = NRC & 7;
   wave_lds_sync();
@@ -946,14 +956,14 @@ __device__ __forceinline__ void dft_subap(const ImageParams& P, const int s, con
     field_trace<N, Q, FULL>(*ray, P.istart[s], P.jstart[s], P.pdiam, lane, fin);
   else
     field_load<N, Q, FULL>(P, win, lane, fin);
-  float inten_scale;
+  int inten_exp;
   dft_spot<N, Q, PREC, FULL, NRC>(P, lane, smem, bin, bm, nr_rt, aw, fin, of, win, unit,
-                                  inten_scale);
+                                  inten_exp);
   wave_lds_sync();
   mid();
   const float I = spot_sum<64>(bin, npix * npix, true, lane);
   void* red = nr > 0 ? smem + spot_f : smem;
-  finish_spot<64, NOISE, KEEP>(P, s, true, lane, bin, I, inten_scale, call_add, red, &pre);
+  finish_spot<64, NOISE, KEEP>(P, s, true, lane, bin, I, inten_exp, call_add, red, &pre);
   wave_lds_sync();
 }
 
@@ -977,19 +987,19 @@ __device__ __forceinline__ void dft_subap_parts(const ImageParams& P, const int 
   const unsigned win = window_corner(P, s);
   FieldIn<Q> fin;
   field_load<N, Q, FULL>(P, win, lane, fin);
-  float inten_scale;
+  int inten_exp;
   dft_spot<N, Q, PREC, FULL, NRC, PARTS>(P, lane, shared, shared, nullptr, NRC & 7, aw, fin, of,
-                                         win, unit, inten_scale, part);
+                                         win, unit, inten_exp, part);
   __syncthreads();  // every kx block binned
   if (part == 0) {
     const float I = spot_sum<64>(shared, npix * npix, true, lane);
-    finish_spot<64, NOISE>(P, s, true, lane, shared, I, inten_scale, call_add, shared + spot_f,
+    finish_spot<64, NOISE>(P, s, true, lane, shared, I, inten_exp, call_add, shared + spot_f,
                            &pre);
   }
 }
 
 // LDS floats per wave of dft_subaps: the |F|^2 image (nr == 0), then SPW
-// spots (16-byte aligned), then SPW spot scales, then 192 doubles for the
+// spots (16-byte aligned), then SPW scale exponents, then 192 doubles for the
 // float64 moment sums of the shared tail.
 template <int N, int Q>
 __host__ __device__ inline int subaps_floats(int npix, bool gather, int spw) {
@@ -1012,7 +1022,7 @@ __device__ __forceinline__ void dft_subaps(const ImageParams& P, const int s0, c
   const int spot_f = (npix2 + 3) & ~3;
   float* hr = smem;
   float* spots = smem + (nr == 0 ? N * N : 0);
-  float* scales = spots + SPW * spot_f;
+  int* exps = reinterpret_cast<int*>(spots + SPW * spot_f);
   // this lane's sub-aperture in the tail: q = lane / 16
   const int q = lane >> 4, r = lane & 15;
   const int s = s0 + q;
@@ -1044,13 +1054,13 @@ __device__ __forceinline__ void dft_subaps(const ImageParams& P, const int s0, c
       for (int k = 0; k < SPW; k += 2) {
         if (s0 + k > last) break;  // uniform
         if (k + 2 < SPW) field_load_pair(P, win[k + 2], win[k + 3], lane, fin[((k >> 1) + 1) & 1]);
-        float scale_a, scale_b;
+        int exp_a, exp_b;
         dft_spot_pair<N, PREC, NRC>(P, lane, spots + k * spot_f, spots + (k + 1) * spot_f, aw,
                                     fin[(k >> 1) & 1], of, win[k], win[k + 1], unit[k],
-                                    unit[k + 1], scale_a, scale_b);
+                                    unit[k + 1], exp_a, exp_b);
         if (lane == 0) {
-          scales[k] = scale_a;
-          scales[k + 1] = scale_b;
+          exps[k] = exp_a;
+          exps[k + 1] = exp_b;
         }
       }
     }
@@ -1061,17 +1071,17 @@ __device__ __forceinline__ void dft_subaps(const ImageParams& P, const int s0, c
     for (int k = 0; k < SPW; ++k) {
       if (s0 + k > last) break;  // uniform
       if (k + 1 < SPW) field_load<N, Q, FULL>(P, win[k + 1], lane, fin[(k + 1) & 1]);
-      float inten_scale;
+      int inten_exp;
       dft_spot<N, Q, PREC, FULL, NRC>(P, lane, hr, spots + k * spot_f, bm, nr_rt, aw, fin[k & 1],
-                                      of, win[k], unit[k], inten_scale);
-      if (lane == 0) scales[k] = inten_scale;
+                                      of, win[k], unit[k], inten_exp);
+      if (lane == 0) exps[k] = inten_exp;
     }
   }
   wave_lds_sync();
   float* sp = spots + q * spot_f;
   const float I = spot_sum<16>(sp, npix2, valid, r);
-  double* red = reinterpret_cast<double*>(scales + ((SPW + 3) & ~3));  // 8-byte aligned
-  finish_spot<16, NOISE>(P, s, valid, r, sp, I, scales[q], call_add, red, &pre);
+  double* red = reinterpret_cast<double*>(exps + ((SPW + 3) & ~3));  // 8-byte aligned
+  finish_spot<16, NOISE>(P, s, valid, r, sp, I, exps[q], call_add, red, &pre);
   wave_lds_sync();
 }
 

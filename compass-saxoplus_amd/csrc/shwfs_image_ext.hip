@@ -355,7 +355,7 @@ void sh_image_ext_kernel(ImageParams P, ExtParams X) {
     float part = 0.0f;
     for (int p = lane; p < npix2; p += 64) part += bin[p];
     const float I = lane_group_sum<64>(part);
-    finish_spot<64, NOISE>(P, s, true, lane, bin, I, 1.0f);
+    finish_spot<64, NOISE>(P, s, true, lane, bin, I, 0);
   }
 }
 

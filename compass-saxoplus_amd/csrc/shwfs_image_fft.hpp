@@ -136,7 +136,7 @@ __device__ __forceinline__ void fft_tile(const ImageParams& P, int s0, float* sm
   tile_sync<TPB>();
 
   // ---- 3. tail
-  spot_tail<N, N, NOISE, KEEP>(P, s, valid, lane, hr, bin, bm, 1.0f, call_add);
+  spot_tail<N, N, NOISE, KEEP>(P, s, valid, lane, hr, bin, bm, 0, call_add);
   tile_sync<TPB>();
 }
 
@@ -214,7 +214,7 @@ __device__ __forceinline__ void fft_wave(const ImageParams& P, int s, int lane, 
   float part = 0.0f;  // fft_tile's sums: N lanes, pixels p, p + N, ... in turn
   for (int p = lane % N; p < npix2; p += N) part += bin[p];
   const float I = lane_group_sum<N>(part);
-  finish_spot<64, true>(P, s, true, lane, bin, I, 1.0f, 0u, nullptr, &pre);
+  finish_spot<64, true>(P, s, true, lane, bin, I, 0, 0u, nullptr, &pre);
 }
 
 }  // namespace shwfs

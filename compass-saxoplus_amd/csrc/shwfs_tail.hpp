@@ -352,7 +352,7 @@ __device__ __forceinline__ float spot_sum(const float* sp, int npix2, bool valid
 
 // Binned spot -> flux normalisation, noise, bincube / binimg, fused
 // centroid.  bin: the npix^2 binned pixels of sub-aperture s in LDS (x
-// fastest), in units of 1/inten_scale; I: their sum (the same units).
+// fastest), in units of 2^-inten_exp; I: their sum (the same units).
 // red: for LANES == 64, LDS scratch of 192 doubles for the moment totals
 // (wave_sum3; must not overlap bin), or nullptr for the DPP reductions.
 // pre: the sub-aperture's scalars loaded beforehand, or nullptr.
@@ -360,14 +360,14 @@ __device__ __forceinline__ float spot_sum(const float* sp, int npix2, bool valid
 // learned centroider, which runs after the tail over several spots).
 template <int LANES, bool NOISE, bool KEEP = false>
 __device__ __forceinline__ void finish_spot(const ImageParams& P, int s, bool valid, int lane,
-                                            float* bin, float I, float inten_scale,
+                                            float* bin, float I, int inten_exp,
                                             unsigned call_add = 0u, void* red = nullptr,
                                             const SubapScalars* pre = nullptr) {
   Moments m;
   if constexpr (KEEP) {
     if (valid) {
       const float fl = pre ? pre->fl : P.flux[s];
-      if (lane == 0) P.intensities[s] = I * inten_scale;
+      if (lane == 0) P.intensities[s] = ldexpf(I, inten_exp);
       const float fnorm = (I != 0.0f) ? fl * __builtin_amdgcn_rcpf(I) * P.nphot : 1.0f;
       const int vx = pre ? pre->vx : P.validsubsx[s];
       const int vy = pre ? pre->vy : P.validsubsy[s];
@@ -384,7 +384,7 @@ __device__ __forceinline__ void finish_spot(const ImageParams& P, int s, bool va
     const float fl = pre ? pre->fl : P.flux[s];
     const int vx = pre ? pre->vx : P.validsubsx[s];
     const int vy = pre ? pre->vy : P.validsubsy[s];
-    if (lane == 0) P.intensities[s] = I * inten_scale;
+    if (lane == 0) P.intensities[s] = ldexpf(I, inten_exp);
     // photometric normalisation b * flux / I * nphot as one factor
     const float fnorm = (I != 0.0f) ? fl * __builtin_amdgcn_rcpf(I) * P.nphot : 1.0f;
     // noise-free 8x8-pixel spots (the usual SH detector) take the fixed-size
@@ -480,17 +480,17 @@ __device__ __forceinline__ float bin_gather(const ImageParams& P, bool valid, in
 }
 
 // hr: the NF x NF |E|^2 image of this sub-aperture in LDS, flat index u + v*NF,
-// holding inten_scale^-1 times the true intensities (a power of two).
+// holding 2^-inten_exp times the true intensities.
 // bin: npix^2 floats of LDS private to this sub-aperture.
 template <int LANES, int NF, bool NOISE, bool KEEP = false>
 __device__ __forceinline__ void spot_tail(const ImageParams& P, int s, bool valid, int lane,
                                           const float* hr, float* bin, const int* s_binmap,
-                                          float inten_scale, unsigned call_add = 0u,
+                                          int inten_exp, unsigned call_add = 0u,
                                           void* red = nullptr,
                                           const SubapScalars* pre = nullptr) {
   const float part = bin_gather<LANES, NF>(P, valid, lane, hr, bin, s_binmap);
   const float I = lane_group_sum<LANES>(part);
-  finish_spot<LANES, NOISE, KEEP>(P, s, valid, lane, bin, I, inten_scale, call_add, red, pre);
+  finish_spot<LANES, NOISE, KEEP>(P, s, valid, lane, bin, I, inten_exp, call_add, red, pre);
 }
 
 }  // namespace shwfs
