@@ -61,7 +61,9 @@ int32_t launch_image_dft(const ImageParams& p, int nfft, int method, hipStream_t
 }
 
 bool split_fp16_fits(const ImageParams& p, int nfft) {
-  return !(p.noise > -1.0f) && p.tpb == 0 && (nfft == 16 || nfft == 32) && p.pdiam <= 16;
+  if (p.noise > -1.0f || p.tpb != 0 || p.pdiam > 16) return false;
+  if (nfft == 32) return p.pdiam >= 5;
+  return nfft == 16 && p.pdiam >= (dft_register_rebin(p) > 0 ? 7 : 9);
 }
 
 int32_t launch_image_split(const ImageParams& p, int nfft, hipStream_t st) {

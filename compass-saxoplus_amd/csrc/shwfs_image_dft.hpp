@@ -26,14 +26,19 @@
 // their error against the float64 oracle.
 //   * kSplitFp16 (no method of its own: how noise-free frames of
 //     SHWFS_METHOD_FFT_FP32 run, split_fp16_fits): every operand x = hi + lo
-//     (fp16 each, 23 significant bits; the power-of-two scales of FP16 keep lo
-//     in range), hi*hi + hi*lo + lo*hi, 3 MFMA per tile, and the field's
-//     float-exact reduction and polynomials (phase_sincos).  For nfft 16 and
-//     32 with windows of up to 16 points.  Relative error of the spots against
-//     float64 over those shapes: 6-11e-8, the in-register FP32 FFT's 6-11e-8
-//     (80x80, nfft 32: 7.8e-8 against 8.8e-8; 40x40, nfft 16: 8.5 against
-//     8.9e-8).  The FFT is bound by its 1,660 VALU instructions per two
-//     sub-apertures; here the transform is on the matrix cores.
+//     (fp16 each), hi*hi + hi*lo + lo*hi, 3 MFMA per tile, and the field's
+//     float-exact reduction and polynomials (phase_sincos).  hi + lo holds x to
+//     2^-23 |x| while lo is a normal fp16.  The power-of-two scales of FP16 see
+//     to that for the table and G; a unit window's field enters unscaled, so a
+//     lo below 2^-14 is a multiple of 2^-24 and small components are held to
+//     2^-25 absolute, a float's rounding near 1.  (Field and table scaled evenly, 2^6 and 2^4,
+//     and the fourth product lo*lo moved no error against float64 by more than
+//     its spread over screens.)  For nfft 16 and 32 with windows of up to 16
+//     points.  Relative error of the spots against float64 over those shapes:
+//     6-11e-8, the in-register FP32 FFT's 6-11e-8 (80x80, nfft 32: 7.8e-8
+//     against 8.8e-8; 40x40, nfft 16: 8.5 against 8.9e-8).  The FFT is bound by
+//     its 1,660 VALU instructions per two sub-apertures; here the transform is
+//     on the matrix cores.
 // Binning, noise, detector image and
 // centroids follow the same definitions as the FFT kernel.
 #pragma once

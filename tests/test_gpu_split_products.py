@@ -1,5 +1,6 @@
-"""Noise-free frames of the FFT method: the split-FP16 products (nfft 16 and
-32, windows of up to 16 points) against the in-register FFT that a named
+"""Noise-free frames of the FFT method: the split-FP16 products (nfft 32,
+windows of 5 to 16 points; nfft 16, 7 to 16, or 9 to 16 with the general
+binmap) against the in-register FFT that a named
 workgroup size selects, and both against the float64 oracle, over every form
 that the products take: each rebin code, the general binmap (nrebin 3), full
 and small windows, one sub-aperture to several workgroups, amplitudes far from
@@ -95,7 +96,7 @@ def test_dark_and_invalid_windows_match_the_fft():
 
 def test_named_workgroup_size_keeps_the_fft():
     """wg_size 64, 128 and 256 all name the in-register FFT (the same bits);
-    the default frame is another computation of the same spots."""
+    the default frame is another computation of the same spots (other bits)."""
     s, _ = _system(8, 16, 32, 4, 8)
     got = []
     for wg in (64, 128, 256, 0):
@@ -103,4 +104,44 @@ def test_named_workgroup_size_keeps_the_fft():
         s.comp_image(noise=False)
         got.append(s.bincube())
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
-    assert relative_array_error(got[3], got[0]) < 1e-6
+    assert 0.0 < relative_array_error(got[3], got[0]) < 1e-6
+
+
+@pytest.mark.parametrize("pd,nfft,nrebin,npix,products", [
+    (6, 16, 2, 8, False), (7, 16, 2, 8, True), (16, 16, 1, 10, True), (8, 16, 3, 5, False),
+    (9, 16, 3, 5, True), (8, 16, 2, 7, False), (9, 16, 2, 7, True), (4, 32, 4, 8, False),
+    (5, 32, 4, 8, True), (5, 32, 3, 9, True), (16, 32, 2, 11, True), (17, 32, 4, 8, False),
+    (16, 64, 4, 8, False)])
+def test_forms_that_take_the_products(pd, nfft, nrebin, npix, products):
+    """Which frames are the FFT's own bits, on both sides of each edge (2x2
+    binning of 7 pixels starts off the block grid: the general binmap)."""
+    s, _ = _system(12, pd, nfft, nrebin, npix)
+    fft, default = _both(s)
+    e = relative_array_error(default[0], fft[0])
+    print("pd %d nfft %d nrebin %d npix %d: %.1e" % (pd, nfft, nrebin, npix, e), flush=True)
+    assert (0.0 < e < 1e-6) if products else all(np.array_equal(a, b)
+                                                 for a, b in zip(fft, default))
+
+
+@pytest.mark.parametrize("pd,nfft,nrebin,npix", [
+    (7, 16, 2, 8), (8, 16, 2, 8), (16, 16, 2, 8), (11, 16, 3, 5), (5, 32, 4, 8), (8, 32, 3, 9),
+    (11, 32, 3, 9), (16, 32, 2, 12), (16, 32, 4, 8)])
+def test_products_are_no_further_off_than_the_fft(pd, nfft, nrebin, npix):
+    """Relative error (2-norm) of spots and flux against the oracle, the mean
+    over 16 screens.  The two errors are of independent roundings: their ratio
+    spreads by 7 % from screen to screen (some 100 sub-apertures each), 1.8 %
+    over 16, so the products' is at most 1.05 times the FFT's."""
+    nx = 12
+    c = configs.sh_config(0.2 * nx, nx, pd, npix, nfft, nrebin, nphot=1000.0,
+                          seeds=range(1, 17))
+    s = system.ShSystem(c)
+    err = np.zeros((2, 2))
+    for phase in system.make_screens(c):
+        s.set_phase(phase)
+        want = _want(s, phase, s.p_geom._mpupil)
+        for k, got in enumerate(_both(s)):
+            for q, (g, w) in enumerate(((got[0], want[0]), (got[2], want[1]))):
+                err[k, q] += np.linalg.norm(g.astype(np.float64) - w) / np.linalg.norm(w) / 16
+    print("pd %d nfft %d nrebin %d: spots %.3e %.3e flux %.3e %.3e"
+          % (pd, nfft, nrebin, err[0, 0], err[1, 0], err[0, 1], err[1, 1]), flush=True)
+    assert np.all(err[1] <= 1.05 * err[0])
