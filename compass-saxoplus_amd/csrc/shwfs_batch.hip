@@ -78,18 +78,19 @@ double tile_cost(const BatchTask& t, int nfft) {
   return (double)t.per_tile * nfft * nfft;
 }
 
-int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, hipStream_t st,
-                  BatchTask* out, size_t* lds) {
+// products: whether the FFT method's default tile of a noise-free batch takes
+// the products that its frames take alone (split_fp16_fits); split 1 or 2 names
+// the in-register FFT.
+int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, bool products,
+                  hipStream_t st, BatchTask* out, size_t* lds) {
   const shwfs_sh_geom& g = b->geoms[i];
   BatchTask t{};
   t.P = b->params[i];
   const int nfft = g.nfft, pdiam = g.nphase, npix = g.npix;
   int32_t rc = check_geom(&g, tile.method);
   if (rc) return rc;
-  // the FFT method's default tile of a noise-free batch: the products that its
-  // frames take alone (split_fp16_fits); split 1 or 2 names the in-register FFT
-  const bool products = tile.method == SHWFS_METHOD_FFT_FP32 && tile.split == 0 && !b->noisy &&
-                        split_fp16_fits(t.P, nfft);
+  products = products && tile.method == SHWFS_METHOD_FFT_FP32 && tile.split == 0 && !b->noisy &&
+             split_fp16_fits(t.P, nfft);
   if (tile.method == SHWFS_METHOD_FFT_FP32 && !products) {
     int split = tile.split;
     if (split == 0) split = 2 * pdiam <= nfft ? 2 : 1;
@@ -242,19 +243,28 @@ bool setup_groups(shwfs_batch* b, std::vector<BatchTask>& tasks, std::vector<dou
   return true;
 }
 
-int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
-  const int n = (int)b->geoms.size();
-  // the table may still be read by frames in flight on any stream
-  SHWFS_HIP(hipDeviceSynchronize());
-  std::vector<BatchTask> tasks(n);
-  std::vector<double> cost(n);
+// Tasks of the batch and the kernel that runs them.
+struct BatchPlan {
+  std::vector<BatchTask> tasks;
+  std::vector<double> cost;
+  std::vector<int> order;  // of a grouped batch
   size_t lds = 0;
+  bool uni = false, grouped = false;
+};
+
+int32_t plan_tasks(shwfs_batch* b, bool products, hipStream_t st, BatchPlan* out) {
+  const int n = (int)b->geoms.size();
+  BatchPlan p;
+  p.tasks.resize(n);
+  p.cost.resize(n);
+  p.order.resize(n);
+  std::vector<BatchTask>& tasks = p.tasks;
   for (int i = 0; i < n; ++i) {
     size_t l = 0;
-    int32_t rc = fill_task(b, i, b->tiles[i], st, &tasks[i], &l);
+    int32_t rc = fill_task(b, i, b->tiles[i], products, st, &tasks[i], &l);
     if (rc) return rc;
-    lds = std::max(lds, l);
-    cost[i] = tile_cost(tasks[i], b->geoms[i].nfft);
+    p.lds = std::max(p.lds, l);
+    p.cost[i] = tile_cost(tasks[i], b->geoms[i].nfft);
   }
   // same-kind MFMA batch (one kind, rebin factor and window class for all, at
   // most kTaskArgs WFS: their parameters travel as kernel arguments): tiles of
@@ -283,22 +293,55 @@ int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
     }
     if (wlds * kDftWaves > max_lds_per_block()) uni = false;
     if (uni) {
-      lds = wlds;
+      p.lds = wlds;
       for (int i = 0; i < n; ++i) {
         tasks[i].per_tile = kDftTaskSubaps;
         tasks[i].ntiles = (b->geoms[i].nvalid + kDftTaskSubaps - 1) / kDftTaskSubaps;
-        cost[i] = tile_cost(tasks[i], b->geoms[i].nfft);
+        p.cost[i] = tile_cost(tasks[i], b->geoms[i].nfft);
       }
     }
   }
-  std::vector<int> order(n);
+  p.uni = uni;
   b->group_kernel = -1;
-  bool grouped = false;
   if (!uni) {
     size_t glds = 0;
-    grouped = setup_groups(b, tasks, cost, order, &glds, st);
-    if (grouped) lds = glds;
+    p.grouped = setup_groups(b, tasks, p.cost, p.order, &glds, st);
+    if (p.grouped) p.lds = glds;
   }
+  *out = std::move(p);
+  return SHWFS_OK;
+}
+
+// The products of the FFT method's default tiles run in the same-kind kernel
+// (register binning) and in the registered group kernels.  Any other batch
+// takes the in-register FFT for them: the general kernel has no stage of
+// theirs, since each call saves registers through scratch and the union of
+// kinds costs more than the products gain.  Per frame, FFT and products (the
+// general kernel with them): two 40x40 of nfft 32 and 64 25.2 and 32.8 us, two
+// 80x80 and an 8x8 of nfft 64 35.4 and 48.4, 40x40 of nrebin 4 and 3 14.1 and
+// 21.2, group kernels of FFT and MFMA stages 20.5-26.5 and 43.5-115; three
+// 40x40 of nrebin 3 (same kind, general binmap) 14.7 and 15.3.
+bool products_fit(const BatchPlan& p) {
+  return p.grouped || (p.uni && p.tasks[0].nr > 0);
+}
+
+int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
+  const int n = (int)b->geoms.size();
+  // the table may still be read by frames in flight on any stream
+  SHWFS_HIP(hipDeviceSynchronize());
+  BatchPlan plan;
+  int32_t rc = plan_tasks(b, true, st, &plan);
+  if (rc) return rc;
+  const auto product = [](const BatchTask& t) { return batch_kind_prec(t.kind) == kSplitFp16; };
+  if (std::any_of(plan.tasks.begin(), plan.tasks.end(), product) && !products_fit(plan)) {
+    rc = plan_tasks(b, false, st, &plan);
+    if (rc) return rc;
+  }
+  const std::vector<BatchTask>& tasks = plan.tasks;
+  const std::vector<double>& cost = plan.cost;
+  std::vector<int>& order = plan.order;
+  const size_t lds = plan.lds;
+  const bool uni = plan.uni, grouped = plan.grouped;
   if (lds > max_lds_per_block())
     return fail(SHWFS_ERR_UNSUPPORTED, "batch: LDS footprint exceeds the per-workgroup limit");
   // waves per workgroup of the mixed kernel: kBatchWaves slots if they fit
@@ -327,10 +370,10 @@ int32_t build_tasks(shwfs_batch* b, hipStream_t st) {
   b->waves = waves;
   int set = 0;
   for (const auto& t : sorted) set |= batch_kind_set(t.kind);
-  b->kind_set = (set & (set - 1)) == 0 ? set : BKS_ALL;  // one set, or all
+  b->kind_set = (set == BKS_FFT || set == BKS_BF16 || set == BKS_FP16) ? set : BKS_ALL;
   b->uni_method = -1;
   if (uni) {
-    b->uni_method = m0;
+    b->uni_method = batch_kind_prec(tasks[0].kind);
     b->uni_nfft = b->geoms[0].nfft;
     b->uni_pdiam = b->geoms[0].nphase;
     b->uni_nr = tasks[0].nr;

@@ -23,7 +23,8 @@ enum BatchKind : int32_t {
   BK_FFT16_1 = 0, BK_FFT16_2, BK_FFT32_1, BK_FFT32_2, BK_FFT64_1, BK_FFT64_2,
   BK_BF16_16, BK_BF16_32, BK_BF16_64, BK_BF16_32Q2, BK_BF16_64Q2,
   BK_FP16_16, BK_FP16_32, BK_FP16_64, BK_FP16_32Q2, BK_FP16_64Q2,
-  // split-FP16: noise-free batches of SHWFS_METHOD_FFT_FP32 with split 0
+  // split-FP16: noise-free batches of SHWFS_METHOD_FFT_FP32 with split 0, in
+  // the same-kind and group kernels only
   BK_SPLIT_16, BK_SPLIT_32,
   BK_COUNT
 };
@@ -95,13 +96,10 @@ __device__ __noinline__ void batch_dft(const BatchTask* task, int s0, unsigned c
 // Kind sets compiled into one batch kernel: the host launches the smallest
 // instantiation that covers the kinds of its tasks (a kernel holding every
 // kind pays for the union of their registers and code size).
-enum BatchKindSet : int { BKS_FFT = 1, BKS_BF16 = 2, BKS_FP16 = 4, BKS_SPLIT = 8, BKS_ALL = 15 };
+enum BatchKindSet : int { BKS_FFT = 1, BKS_BF16 = 2, BKS_FP16 = 4, BKS_ALL = 7 };
 
 __host__ __device__ constexpr int batch_kind_set(int kind) {
-  return kind < BK_BF16_16    ? BKS_FFT
-         : kind < BK_FP16_16  ? BKS_BF16
-         : kind < BK_SPLIT_16 ? BKS_FP16
-                              : BKS_SPLIT;
+  return kind < BK_BF16_16 ? BKS_FFT : (kind < BK_FP16_16 ? BKS_BF16 : BKS_FP16);
 }
 
 // slot: LDS floats per wave (the largest slot of the tasks); launched with
@@ -172,12 +170,6 @@ void sh_batch_kernel(const BatchTask* __restrict__ tasks, const TaskStarts start
         break;
       case BK_FP16_64Q2:
         if constexpr ((SET & BKS_FP16) != 0) batch_dft<64, 2, SHWFS_METHOD_DFT_FP16, NOISE>(&T, s0, fcall, slot);
-        break;
-      case BK_SPLIT_16:
-        if constexpr ((SET & BKS_SPLIT) != 0 && !NOISE) batch_dft<16, 1, kSplitFp16, false>(&T, s0, fcall, slot);
-        break;
-      case BK_SPLIT_32:
-        if constexpr ((SET & BKS_SPLIT) != 0 && !NOISE) batch_dft<32, 1, kSplitFp16, false>(&T, s0, fcall, slot);
         break;
       default: break;
     }

@@ -24,7 +24,6 @@ int32_t launch_batch_quiet(int set, const BatchTask* tasks, const TaskStarts& st
     case BKS_FFT: return launch_set<BKS_FFT>(tasks, starts, ntasks, total_tiles, grid, waves, lds, frame_base, frame_off, remap, st);
     case BKS_BF16: return launch_set<BKS_BF16>(tasks, starts, ntasks, total_tiles, grid, waves, lds, frame_base, frame_off, remap, st);
     case BKS_FP16: return launch_set<BKS_FP16>(tasks, starts, ntasks, total_tiles, grid, waves, lds, frame_base, frame_off, remap, st);
-    case BKS_SPLIT: return launch_set<BKS_SPLIT>(tasks, starts, ntasks, total_tiles, grid, waves, lds, frame_base, frame_off, remap, st);
     default: return launch_set<BKS_ALL>(tasks, starts, ntasks, total_tiles, grid, waves, lds, frame_base, frame_off, remap, st);
   }
 }
@@ -43,7 +42,6 @@ int batch_blocks_per_cu_quiet(int set, int waves, size_t lds) {
     case BKS_FFT: return occupancy<BKS_FFT>(waves, lds);
     case BKS_BF16: return occupancy<BKS_BF16>(waves, lds);
     case BKS_FP16: return occupancy<BKS_FP16>(waves, lds);
-    case BKS_SPLIT: return occupancy<BKS_SPLIT>(waves, lds);
     default: return occupancy<BKS_ALL>(waves, lds);
   }
 }

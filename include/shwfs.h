@@ -423,11 +423,15 @@ typedef struct shwfs_batch shwfs_batch; /* opaque */
 typedef struct shwfs_batch_tile {
   int32_t method; /* SHWFS_METHOD_* used for this WFS in the batch */
   int32_t split;  /* FFT method: 1, or 2 (row transforms split in two, needs
-                     2*nphase <= nfft); 0 = the split-FP16 products where a
-                     noise-free batch allows them (as SHWFS_METHOD_FFT_FP32),
-                     else 2 when allowed.  Ignored by DFT. */
+                     2*nphase <= nfft); 0 = the split-FP16 products of the frame
+                     alone (SHWFS_METHOD_FFT_FP32) in a noise-free batch whose
+                     WFS are of one kind with binning blocks of 1, 2 or 4, or the
+                     mix of the uneven-batch kernels, else 2 when allowed.
+                     Ignored by DFT. */
 } shwfs_batch_tile;
-/* frames[i].method is the initial method of WFS i (wg_size is ignored).
+/* frames[i].method is the initial method of WFS i; a wg_size other than 0
+ * names the in-register FFT of the FFT method, as in a frame alone, and no
+ * workgroup size.
  * Refused (SHWFS_ERR_UNSUPPORTED): ntot != nfft, kernconv, LGS kernels, layers, and the
  * SHWFS_CENTROID_MLP kind, which run per WFS through shwfs_sh_comp_image. */
 int32_t shwfs_batch_create(const shwfs_sh_geom* geoms, const shwfs_frame_args* frames,
