@@ -24,9 +24,11 @@ constexpr int TS = 32;          // samples per tile
 constexpr int TPB = 256;        // 4 waves
 using Lds = mlp::Lds<TS>;
 constexpr size_t LDS_BYTES = Lds::bytes();
-// work buffer: bf16 copies of W1 and W2 (inference), or W1, W2 and W2^T as
-// MFMA operands, then the workgroups' partial gradients (gradient)
-constexpr size_t WORK_ELEMS = (size_t)NH * NIN + 2 * (size_t)NH * NH;
+// work buffer: bf16 copies of W1 and W2 (inference), then W1, W2 and W2^T as
+// MFMA operands (gradient): a function of the parameters alone, so that calls
+// with the same parameters on several streams may share one
+constexpr size_t kInferElems = (size_t)NH * NIN + (size_t)NH * NH;
+constexpr size_t WORK_ELEMS = kInferElems + (size_t)NH * NIN + 2 * (size_t)NH * NH;
 
 // X tile of samples row0 .. row0+TS-1 (rows >= rows_valid zero) -> bf16 in LDS.
 __device__ void load_rows(const float* __restrict__ x, long row0, int rows_valid, float x_scale,
@@ -86,13 +88,14 @@ __global__ __launch_bounds__(TPB) void mlp_tile_kernel(const float* __restrict__
 constexpr int kGradWaves = 8;
 constexpr int kGradThreads = 64 * kGradWaves;
 constexpr int kGradStep = 16 * kGradWaves;  // samples of a step
-constexpr int kGradMaxGroups = 256;         // one workgroup per CU (149 KiB of LDS)
-// Up to kGradAtomicGroups workgroups add their sums to the gradient by
-// atomics; more of them store partial gradients that a second kernel sums.
-// Whole calls at 32,768 samples (256 workgroups): 75 us with atomics, 56 with
-// partial sums; at 4,096 (32 workgroups) 45.7 and 44.8: no gain for the work
-// space there.
-constexpr int kGradAtomicGroups = 32;
+constexpr int kGradMaxGroups = 256;         // one workgroup per CU (153 KiB of LDS)
+// Up to kGradAtomicGroups workgroups, or without a buffer for partial
+// gradients, the workgroups add their sums to the gradient by atomics; else
+// they store partial gradients that a second kernel sums.  Whole calls with
+// atomics and with partial sums: 4,200 samples (33 workgroups) 38.0 and 40.2
+// us, 8,000 (63) 40.6 and 42.9, 16,384 (128) 47.2 and 44.8, 32,768 (256) 59.8
+// and 51.0, 131,072 (256) 90.5 and 78.5.
+constexpr int kGradAtomicGroups = 64;
 constexpr int kGradSlot = NPARAM + 2;       // partial gradient, loss, padding (16-byte rows)
 constexpr int kGradSplit = 8;               // workgroups that share the sum of an element
 constexpr int SS = kGradStep + 8;           // LDS row of samples (16-byte aligned rows)
@@ -108,7 +111,7 @@ __global__ __launch_bounds__(TPB) void mlp_prepare_grad_kernel(const float* __re
                                                                __bf16* __restrict__ work,
                                                                float* __restrict__ grad,
                                                                float* __restrict__ loss) {
-  __bf16* W1f = work;
+  __bf16* W1f = work + kInferElems;
   __bf16* W2f = W1f + kFragW1;
   __bf16* W2tf = W2f + kFragW2;
   for (int i = blockIdx.x * TPB + threadIdx.x; i < NPARAM; i += gridDim.x * TPB) {
@@ -228,9 +231,9 @@ void mlp_grad_kernel(const float* __restrict__ P, const __bf16* __restrict__ wor
   float* sum = sW3 + NOUT * NH;  // db1, db2, dW3 (2), db3, loss
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 15, g = lane >> 4;
-  const __bf16* W1f = work;
+  const __bf16* W1f = work + kInferElems;
   for (int i = tid; i < 2 * kFragW2 / 8; i += kGradThreads)
-    reinterpret_cast<float4*>(sW2)[i] = reinterpret_cast<const float4*>(work + kFragW1)[i];
+    reinterpret_cast<float4*>(sW2)[i] = reinterpret_cast<const float4*>(W1f + kFragW1)[i];
   if (tid < NH) {
     sB1[tid] = P[OB1 + tid];
     sB2[tid] = P[OB2 + tid];
@@ -424,23 +427,24 @@ void mlp_grad_kernel(const float* __restrict__ P, const __bf16* __restrict__ wor
     }
   }
   __syncthreads();
-  float* slot = PART ? grad + (size_t)blockIdx.x * kGradSlot : grad;
-  auto emit = [&](int i, float v) {
-    if constexpr (PART)
-      slot[i] = v;
-    else
-      atomicAdd(&slot[i], v);
-  };
+  // the workgroup's gradient in the parameters' order: to its slot, or over the
+  // operands in LDS, from where it is added 64 consecutive floats per wave, each
+  // workgroup from another element on (added as the accumulators lie, in runs of
+  // 16 and all workgroups in one order: 75 us at 32,768 samples, 60 so)
+  float* out = PART ? grad + (size_t)blockIdx.x * kGradSlot : reinterpret_cast<float*>(smem_raw);
+  static_assert(sizeof(float) * NPARAM <= 2 * sizeof(__bf16) * (size_t)kFragW2 +
+                                              sizeof(__bf16) * (size_t)SS * (2 * NH + NIN),
+                "mlp_grad_kernel: the gradient lies over the operands");
   if (tid < NH) {
-    emit(OB1 + tid, sum[tid]);
-    emit(OB2 + tid, sum[NH + tid]);
-    emit(OW3 + tid, sum[2 * NH + tid]);
-    emit(OW3 + NH + tid, sum[3 * NH + tid]);
-    if (tid < NOUT) emit(OB3 + tid, sum[4 * NH + tid]);
+    out[OB1 + tid] = sum[tid];
+    out[OB2 + tid] = sum[NH + tid];
+    out[OW3 + tid] = sum[2 * NH + tid];
+    out[OW3 + NH + tid] = sum[3 * NH + tid];
+    if (tid < NOUT) out[OB3 + tid] = sum[4 * NH + tid];
     if (tid == NOUT) {
       const float l = sum[4 * NH + 2] / (float)(n * NOUT);
       if constexpr (PART)
-        slot[NPARAM] = l;
+        out[NPARAM] = l;
       else
         atomicAdd(loss, l);
     }
@@ -448,11 +452,22 @@ void mlp_grad_kernel(const float* __restrict__ P, const __bf16* __restrict__ wor
 #pragma unroll
   for (int nt = 0; nt < 8; ++nt)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) emit(OW2 + (16 * w + 4 * g + v) * NH + 16 * nt + j, a2[nt][v]);
+    for (int v = 0; v < 4; ++v) out[OW2 + (16 * w + 4 * g + v) * NH + 16 * nt + j] = a2[nt][v];
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) emit(OW1 + (16 * w + 4 * g + v) * NIN + 16 * nt + j, a1[nt][v]);
+    for (int v = 0; v < 4; ++v) out[OW1 + (16 * w + 4 * g + v) * NIN + 16 * nt + j] = a1[nt][v];
+  if constexpr (!PART) {
+    __syncthreads();
+    constexpr int kChunks = (NPARAM + kGradThreads - 1) / kGradThreads;
+    int c = (int)(blockIdx.x % kChunks);
+#pragma unroll 10
+    for (int k = 0; k < kChunks; ++k) {
+      const int i = c * kGradThreads + tid;
+      if (i < NPARAM) atomicAdd(&grad[i], out[i]);
+      c = c + 1 == kChunks ? 0 : c + 1;
+    }
+  }
 }
 
 __global__ __launch_bounds__(TPB) void mlp_adam_kernel(float* __restrict__ P, float* __restrict__ G,
@@ -545,9 +560,9 @@ using namespace shwfs;
 
 extern "C" {
 
-size_t shwfs_mlp_work_bytes(void) {
-  return WORK_ELEMS * sizeof(__bf16) + sizeof(float) * (size_t)kGradMaxGroups * kGradSlot;
-}
+size_t shwfs_mlp_work_bytes(void) { return WORK_ELEMS * sizeof(__bf16); }
+
+size_t shwfs_mlp_part_bytes(void) { return sizeof(float) * (size_t)kGradMaxGroups * kGradSlot; }
 
 int32_t shwfs_phase_window(const float* d_src, int32_t src_side, int32_t ox, int32_t oy,
                            float gain, float* d_dst, int32_t n, void* stream) {
@@ -588,6 +603,14 @@ int32_t shwfs_mlp_forward(const float* d_params, void* d_work, const float* d_x,
 int32_t shwfs_mlp_loss_grad(const float* d_params, void* d_work, const float* d_x,
                             const float* d_t, const int32_t* d_index, int64_t n, float x_scale,
                             float t_scale, float* d_grad, float* d_loss, void* stream) {
+  return shwfs_mlp_loss_grad_part(d_params, d_work, nullptr, d_x, d_t, d_index, n, x_scale,
+                                  t_scale, d_grad, d_loss, stream);
+}
+
+int32_t shwfs_mlp_loss_grad_part(const float* d_params, void* d_work, void* d_part,
+                                 const float* d_x, const float* d_t, const int32_t* d_index,
+                                 int64_t n, float x_scale, float t_scale, float* d_grad,
+                                 float* d_loss, void* stream) {
   if (!d_params || !d_work || !d_x || !d_t || !d_grad || !d_loss)
     return fail(SHWFS_ERR_ARG, "mlp_loss_grad: NULL argument");
   if (n <= 0) return fail(SHWFS_ERR_ARG, "mlp_loss_grad: n must be positive");
@@ -599,13 +622,12 @@ int32_t shwfs_mlp_loss_grad(const float* d_params, void* d_work, const float* d_
   SHWFS_LAUNCHED("mlp_prepare_grad_kernel");
   const int64_t steps = (n + kGradStep - 1) / kGradStep;
   const unsigned grid = (unsigned)(steps < kGradMaxGroups ? steps : kGradMaxGroups);
-  float* part = reinterpret_cast<float*>(static_cast<char*>(d_work) + WORK_ELEMS * sizeof(__bf16));
-  const bool atomics = grid <= (unsigned)kGradAtomicGroups;
-  hipLaunchKernelGGL(atomics ? mlp_grad_kernel<false> : mlp_grad_kernel<true>, dim3(grid),
+  float* part = grid > (unsigned)kGradAtomicGroups ? static_cast<float*>(d_part) : nullptr;
+  hipLaunchKernelGGL(part ? mlp_grad_kernel<true> : mlp_grad_kernel<false>, dim3(grid),
                      dim3(kGradThreads), GRAD_LDS, st, d_params, (const __bf16*)d_work, d_x, d_t,
-                     d_index, (long)n, x_scale, t_scale, atomics ? d_grad : part, d_loss);
+                     d_index, (long)n, x_scale, t_scale, part ? part : d_grad, d_loss);
   SHWFS_LAUNCHED("mlp_grad_kernel");
-  if (!atomics) {
+  if (part) {
     hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3((NPARAM + TPB) / TPB, kGradSplit), dim3(TPB), 0,
                        st, part, (int)grid, d_grad, d_loss);
     SHWFS_LAUNCHED("mlp_grad_sum_kernel");

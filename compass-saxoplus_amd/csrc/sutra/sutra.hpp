@@ -594,6 +594,7 @@ class SutraCentroiderMlp : public SutraCentroider<Tin, T> {
   CarmaObj<float>* d_m;       // Adam moments
   CarmaObj<float>* d_v;
   CarmaObj<float>* d_work;    // bf16 weight copies
+  CarmaObj<float>* d_part;    // partial gradients, or NULL until a large batch is differentiated
   CarmaObj<float>* d_loss;
   CarmaObj<int32_t>* d_fallback;  // [nvalid] 1 where the CoG was used
   float x_scale;              // input scale (1 / photons per sub-aperture)
@@ -621,6 +622,9 @@ class SutraCentroiderMlp : public SutraCentroider<Tin, T> {
   // not fusable into the spot kernel: NONE (comp_frame runs spots then get_cog)
   shwfs_centroid_args centroid_args(float* intensities, T* slopes, int32_t nvalid, int32_t npix,
                                     int32_t size) override;
+
+ private:
+  float* partials(int64_t n);  // d_part for a gradient of n samples
 };
 
 // Training pairs generated by the WFS itself: for each of nframes frames, a

@@ -17,6 +17,7 @@ SutraCentroiderMlp<Tin, T>::SutraCentroiderMlp(CarmaContext* context, SutraWfs* 
       flux_lo(-INFINITY),
       flux_hi(INFINITY),
       step(0) {
+  d_part = nullptr;
   int64_t d[2] = {1, SHWFS_MLP_NPARAM};
   d_params = new CarmaObj<float>(context, d);
   d_grad = new CarmaObj<float>(context, d);
@@ -42,6 +43,7 @@ SutraCentroiderMlp<Tin, T>::~SutraCentroiderMlp() {
   delete d_m;
   delete d_v;
   delete d_work;
+  delete d_part;
   delete d_loss;
   delete d_fallback;
 }
@@ -77,14 +79,26 @@ static void check_xt(CarmaObj<float>* x, CarmaObj<float>* t, int64_t n) {
   if (t && t->get_nb_elements() < n * 2) throw std::invalid_argument("mlp: t smaller than n x 2");
 }
 
+// Objects that only infer, or train on small batches, never hold the 26 MB.
+template <class Tin, class T>
+float* SutraCentroiderMlp<Tin, T>::partials(int64_t n) {
+  constexpr int64_t kLarge = 8192;  // samples from which shwfs_mlp_loss_grad_part uses them
+  if (n <= kLarge) return nullptr;
+  if (!d_part) {
+    int64_t d[2] = {1, (int64_t)(shwfs_mlp_part_bytes() / sizeof(float))};
+    d_part = new CarmaObj<float>(this->current_context, d);
+  }
+  return d_part->get_data();
+}
+
 template <class Tin, class T>
 float SutraCentroiderMlp<Tin, T>::loss_grad(CarmaObj<float>* x, CarmaObj<float>* t, int64_t n,
                                             float t_scale) {
   check_xt(x, t, n);
   this->current_context->set_active_device(this->device, 1);
-  shwfs_throw_if(shwfs_mlp_loss_grad(d_params->get_data(), d_work->get_data(), x->get_data(),
-                                     t->get_data(), nullptr, n, x_scale, t_scale,
-                                     d_grad->get_data(), d_loss->get_data(), nullptr),
+  shwfs_throw_if(shwfs_mlp_loss_grad_part(d_params->get_data(), d_work->get_data(), partials(n),
+                                          x->get_data(), t->get_data(), nullptr, n, x_scale,
+                                          t_scale, d_grad->get_data(), d_loss->get_data(), nullptr),
                  "mlp loss_grad");
   float l = 0.f;
   d_loss->device2host(&l);
@@ -123,10 +137,11 @@ float SutraCentroiderMlp<Tin, T>::train(CarmaObj<float>* x, CarmaObj<float>* t, 
     std::shuffle(perm.begin(), perm.end(), rng);
     d_idx.host2device(perm.data());
     for (int64_t b = 0; b < nb; ++b) {
-      shwfs_throw_if(shwfs_mlp_loss_grad(d_params->get_data(), d_work->get_data(), x->get_data(),
-                                         t->get_data(), d_idx.get_data() + b * batch, batch,
-                                         x_scale, t_scale, d_grad->get_data(),
-                                         d_losses.get_data() + b, nullptr),
+      shwfs_throw_if(shwfs_mlp_loss_grad_part(d_params->get_data(), d_work->get_data(),
+                                              partials(batch), x->get_data(), t->get_data(),
+                                              d_idx.get_data() + b * batch, batch, x_scale,
+                                              t_scale, d_grad->get_data(),
+                                              d_losses.get_data() + b, nullptr),
                      "mlp train");
       ++step;
       shwfs_throw_if(shwfs_mlp_adam(d_params->get_data(), d_grad->get_data(), d_m->get_data(),

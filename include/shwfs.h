@@ -469,8 +469,8 @@ int32_t shwfs_batch_autotune(shwfs_batch* batch, uint32_t method_mask, int32_t r
  * matrix cores, FP32 accumulation, FP32 master parameters.
  * d_params: flat [SHWFS_MLP_NPARAM] = W1 (128x64 row-major), b1 (128),
  * W2 (128x128), b2 (128), W3 (2x128), b3 (2).  d_work: shwfs_mlp_work_bytes()
- * of device scratch for the bf16 weight copies and shwfs_mlp_loss_grad's
- * partial gradients (one call at a time uses it).  Inputs x: [n][64] spots
+ * of device scratch for the bf16 weight copies (calls with the same parameters
+ * may share it, on any streams).  Inputs x: [n][64] spots
  * (pixel px + 8*py), multiplied by x_scale; outputs / targets [n][2] in
  * pixels.  Loss: mean over samples and outputs of (y - t)^2. */
 #define SHWFS_MLP_NPARAM 25090
@@ -485,6 +485,16 @@ int32_t shwfs_mlp_forward(const float* d_params, void* d_work, const float* d_x,
 int32_t shwfs_mlp_loss_grad(const float* d_params, void* d_work, const float* d_x,
                             const float* d_t, const int32_t* d_index, int64_t n, float x_scale,
                             float t_scale, float* d_grad, float* d_loss, void* stream);
+/* The same with d_part: shwfs_mlp_part_bytes() of device scratch that, like
+ * d_grad, belongs to this call alone until it has run, or NULL (as
+ * shwfs_mlp_loss_grad).  With it the workgroups of large batches (over 8,192
+ * samples) store partial gradients that a second kernel sums, faster than
+ * atomics on d_grad. */
+size_t shwfs_mlp_part_bytes(void);
+int32_t shwfs_mlp_loss_grad_part(const float* d_params, void* d_work, void* d_part,
+                                 const float* d_x, const float* d_t, const int32_t* d_index,
+                                 int64_t n, float x_scale, float t_scale, float* d_grad,
+                                 float* d_loss, void* stream);
 /* One Adam step (step >= 1, bias-corrected) on d_params; zeroes d_grad. */
 int32_t shwfs_mlp_adam(float* d_params, float* d_grad, float* d_m, float* d_v, int32_t step,
                        float lr, float beta1, float beta2, float eps, void* stream);
