@@ -128,17 +128,20 @@ __global__ __launch_bounds__(TPB) void mlp_prepare_grad_kernel(const float* __re
   if (blockIdx.x == 0 && threadIdx.x == 0) loss[0] = 0.0f;
 }
 
-// gelu(z) and gelu'(z) from one exponential: with s = 1 / (1 + exp(-2 u)), u =
-// c (z + 0.044715 z^3), (1 + tanh u) / 2 = s and (1 - tanh^2 u) / 4 = s (1 - s).
-// Relative error of s about 3e-7 for every z (1 + tanhf loses its relative
-// accuracy below z = 0).
+// gelu(z) and gelu'(z) from one exponential: with ex = exp(-2 u), u = c (z +
+// 0.044715 z^3), and s = 1 / (1 + ex): (1 + tanh u) / 2 = s and (1 - tanh^2 u)
+// / 4 = s (1 - s), 1 - s = ex s (1 - s itself loses its relative accuracy above
+// z = 0).  Largest errors against float64 over |z| < 6, exp and reciprocal a
+// unit off: gelu 7.7e-7 (the tanhf form 5.8e-7), gelu' 2.9e-7 (3.3e-6); bf16
+// operands round them to 4e-3.  Where ex overflows s is 0 and 1 - s is 1
+// (fminf passes over the NaN of inf 0).
 __device__ __forceinline__ void gelu_both(float z, float& g, float& dg) {
   constexpr float k2 = 2.0f * kGeluC, kA = 0.044715f, kLog2e = 1.44269504088896341f;
   const float z2 = z * z;
-  const float w = z * fmaf(k2 * kA, z2, k2);  // 2 u
-  const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2e * w));
+  const float ex = __builtin_amdgcn_exp2f(z * fmaf(-kLog2e * k2 * kA, z2, -kLog2e * k2));
+  const float s = __builtin_amdgcn_rcpf(1.0f + ex);
   g = z * s;
-  dg = fmaf(g * (1.0f - s), fmaf(3.0f * k2 * kA, z2, k2), s);
+  dg = fmaf(g * fminf(ex * s, 1.0f), fmaf(3.0f * k2 * kA, z2, k2), s);
 }
 
 // Sums over the 16 lanes of a row of the 16 values v: lane j receives the
