@@ -32,6 +32,14 @@ struct RayParams {
   int nx, ny;  // source screen
 };
 
+// Truncation to a grid index, as the hardware takes it: saturated outside int's
+// range, 0 for NaN (a C++ conversion is undefined there).
+__device__ __forceinline__ int grid_index(float x) {
+  int i;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(x));
+  return i;
+}
+
 // Value layer l adds at source point (x, y).  No contraction into fused
 // multiply-adds: the stand-alone and the fused kernels give the same bits.
 __device__ __forceinline__ float ray_layer(const RayLayer& l, int nx, int ny, int x, int y) {
@@ -43,8 +51,9 @@ __device__ __forceinline__ float ray_layer(const RayLayer& l, int nx, int ny, in
   const float y2 = ((l.s * x1 + l.c * y1) + hy) + l.yoff_d;
   const float xref = x2 * l.delta + l.dx;
   const float yref = y2 * l.delta + l.dy;
-  const int i = (int)xref, j = (int)yref;  // truncation, as the reference
-  if (i < 0 || j < 0 || i + 1 >= l.dim || j + 1 >= l.dim) return 0.0f;
+  const int i = grid_index(xref), j = grid_index(yref);  // truncation, as the reference
+  // (i + 1 would overflow at a saturated index; dim >= 2)
+  if (i < 0 || j < 0 || i >= l.dim - 1 || j >= l.dim - 1) return 0.0f;
   const float u = xref - (float)i, v = yref - (float)j;
   const float wx1 = 1.0f - u, wx2 = u, wy1 = 1.0f - v, wy2 = v;
   const float* p = l.screen + (size_t)i + (size_t)j * (size_t)l.dim;
@@ -68,7 +77,7 @@ __device__ __forceinline__ void ray_axis(const RayLayer& l, float h, float off, 
 #pragma clang fp contract(off)
   const float t2 = (((float)t - h) * l.G + h) + off;
   const float ref = t2 * l.delta + d;
-  i = (int)ref;
+  i = grid_index(ref);
   u = ref - (float)i;
 }
 
@@ -96,8 +105,9 @@ __device__ __forceinline__ void ray_points4(const RayParams& R, int l0, int x, i
 #pragma unroll
     for (int e = 0; e < 4; ++e) ray_axis(l, hx, l.xoff_d, l.dx, x + e, i[e], u[k][e]);
     ray_axis(l, hy, l.yoff_d, l.dy, y, j, v[k]);
-    fast = fast && l.axis != 0 && i[1] == i[0] + 1 && i[2] == i[0] + 2 && i[3] == i[0] + 3 &&
-           i[0] >= 0 && i[3] + 1 < l.dim && j >= 0 && j + 1 < l.dim;
+    const unsigned i0 = (unsigned)i[0];
+    fast = fast && l.axis != 0 && (unsigned)i[1] == i0 + 1u && (unsigned)i[2] == i0 + 2u &&
+           (unsigned)i[3] == i0 + 3u && i[0] >= 0 && i[3] < l.dim - 1 && j >= 0 && j < l.dim - 1;
     p[k] = l.screen + (size_t)i[0] + (size_t)j * (size_t)l.dim;
   }
   if (__all(fast)) {

@@ -45,3 +45,36 @@ def test_traced_equals_rendered(nlayers, pd, nfft, G, theta, edge):
                                                                s.wfs.nvalid), flush=True)
     for a, b in zip(*got):
         assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("xo,yo", [(3e9, 5.0), (5.0, 3e9), (-3e9, 5.0), (5.0, -3e9), (3e9, 3e9),
+                                   (float("inf"), 5.0), (5.0, float("inf"))])
+@pytest.mark.parametrize("theta", [0.0, 0.2])
+def test_layers_past_the_index_range_add_nothing(xo, yo, theta):
+    """A layer shifted further than an int holds: no point falls on it."""
+    c = configs.sh_config(0.2 * 10, 10, 16, 4, 32, 2, nphot=1000.0)
+    c["p_wfs"].thetaML = theta
+    s = system.ShSystem(c)
+    n = s.p_geom._n
+    dim = n + 60
+    z = np.zeros(2, np.float32)
+    at = s.sutra.Atmos(s.ctx, 2, 0.16, z + 10, np.full(2, dim, np.int64), np.full(2, 4, np.int64),
+                       z, z, z, z, z, 0)
+    rng = np.random.default_rng(4)
+    for k in range(2):
+        at.d_screens[k].d_screen.host2device(
+            np.asfortranarray(rng.standard_normal((dim, dim)).astype(np.float32)))
+    gs = s.wfs.d_gs
+    gs.add_layer("atmos", 0, 30.25, 29.5)
+    got = []
+    for lazy in (True, False):
+        gs.lazy_raytrace = lazy
+        gs.raytrace(at)
+        s.comp_image(noise=False)
+        got.append(s.bincube())
+    gs.add_layer("atmos", 1, xo, yo)
+    for lazy, want in zip((True, False), got):
+        gs.lazy_raytrace = lazy
+        gs.raytrace(at)
+        s.comp_image(noise=False)
+        assert np.isfinite(want).all() and np.array_equal(s.bincube(), want)
