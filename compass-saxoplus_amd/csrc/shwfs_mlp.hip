@@ -129,12 +129,12 @@ __global__ __launch_bounds__(TPB) void mlp_prepare_grad_kernel(const float* __re
 }
 
 // gelu(z) and gelu'(z) from one exponential: with ex = exp(-2 u), u = c (z +
-// 0.044715 z^3), and s = 1 / (1 + ex): (1 + tanh u) / 2 = s and (1 - tanh^2 u)
-// / 4 = s (1 - s), 1 - s = ex s (1 - s itself loses its relative accuracy above
-// z = 0).  Largest errors against float64 over |z| < 6, exp and reciprocal a
-// unit off: gelu 7.7e-7 (the tanhf form 5.8e-7), gelu' 2.9e-7 (3.3e-6); bf16
-// operands round them to 4e-3.  Where ex overflows s is 0 and 1 - s is 1
-// (fminf passes over the NaN of inf 0).
+// 0.044715 z^3), and s = 1 / (1 + ex), (1 + tanh u) / 2 = s and (1 - tanh^2 u)
+// / 4 = s (1 - s), where 1 - s = ex s (the subtraction loses its relative
+// accuracy above z = 0).  Largest errors against float64 over |z| < 6, exp and
+// reciprocal a unit off: gelu 7.7e-7 (the tanhf form 5.8e-7), gelu' 2.9e-7
+// (3.3e-6); bf16 rounds the operands made of them to 2e-3.  Where ex overflows
+// s is 0 and 1 - s is 1 (fminf passes over the NaN of inf times 0).
 __device__ __forceinline__ void gelu_both(float z, float& g, float& dg) {
   constexpr float k2 = 2.0f * kGeluC, kA = 0.044715f, kLog2e = 1.44269504088896341f;
   const float z2 = z * z;

@@ -624,7 +624,7 @@ class SutraCentroiderMlp : public SutraCentroider<Tin, T> {
                                     int32_t size) override;
 
  private:
-  float* partials(int64_t n);  // d_part for a gradient of n samples
+  void alloc_partials(int64_t n);  // d_part, where a gradient of n samples uses it
 };
 
 // Training pairs generated by the WFS itself: for each of nframes frames, a

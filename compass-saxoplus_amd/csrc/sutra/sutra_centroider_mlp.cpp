@@ -81,14 +81,11 @@ static void check_xt(CarmaObj<float>* x, CarmaObj<float>* t, int64_t n) {
 
 // Objects that only infer, or train on small batches, never hold the 26 MB.
 template <class Tin, class T>
-float* SutraCentroiderMlp<Tin, T>::partials(int64_t n) {
-  constexpr int64_t kLarge = 8192;  // samples from which shwfs_mlp_loss_grad_part uses them
-  if (n <= kLarge) return nullptr;
-  if (!d_part) {
-    int64_t d[2] = {1, (int64_t)(shwfs_mlp_part_bytes() / sizeof(float))};
-    d_part = new CarmaObj<float>(this->current_context, d);
-  }
-  return d_part->get_data();
+void SutraCentroiderMlp<Tin, T>::alloc_partials(int64_t n) {
+  constexpr int64_t kLarge = 8192;  // samples past which shwfs_mlp_loss_grad_part uses them
+  if (n <= kLarge || d_part) return;
+  int64_t d[2] = {1, (int64_t)(shwfs_mlp_part_bytes() / sizeof(float))};
+  d_part = new CarmaObj<float>(this->current_context, d);
 }
 
 template <class Tin, class T>
@@ -96,10 +93,12 @@ float SutraCentroiderMlp<Tin, T>::loss_grad(CarmaObj<float>* x, CarmaObj<float>*
                                             float t_scale) {
   check_xt(x, t, n);
   this->current_context->set_active_device(this->device, 1);
-  shwfs_throw_if(shwfs_mlp_loss_grad_part(d_params->get_data(), d_work->get_data(), partials(n),
-                                          x->get_data(), t->get_data(), nullptr, n, x_scale,
-                                          t_scale, d_grad->get_data(), d_loss->get_data(), nullptr),
+  shwfs_throw_if(shwfs_mlp_loss_grad_part(d_params->get_data(), d_work->get_data(),
+                                          d_part ? d_part->get_data() : nullptr, x->get_data(),
+                                          t->get_data(), nullptr, n, x_scale, t_scale,
+                                          d_grad->get_data(), d_loss->get_data(), nullptr),
                  "mlp loss_grad");
+  alloc_partials(n);  // for the next call, while this one runs (70 us of hipMalloc)
   float l = 0.f;
   d_loss->device2host(&l);
   return l;
@@ -132,13 +131,15 @@ float SutraCentroiderMlp<Tin, T>::train(CarmaObj<float>* x, CarmaObj<float>* t, 
   if (nb == 0) throw std::invalid_argument("mlp train: fewer pairs than one batch");
   int64_t dl[2] = {1, nb};
   CarmaObj<float> d_losses(this->current_context, dl);
+  alloc_partials(batch);
   float last = 0.f;
   for (int32_t e = 0; e < epochs; ++e) {
     std::shuffle(perm.begin(), perm.end(), rng);
     d_idx.host2device(perm.data());
     for (int64_t b = 0; b < nb; ++b) {
       shwfs_throw_if(shwfs_mlp_loss_grad_part(d_params->get_data(), d_work->get_data(),
-                                              partials(batch), x->get_data(), t->get_data(),
+                                              d_part ? d_part->get_data() : nullptr,
+                                              x->get_data(), t->get_data(),
                                               d_idx.get_data() + b * batch, batch, x_scale,
                                               t_scale, d_grad->get_data(),
                                               d_losses.get_data() + b, nullptr),

@@ -120,3 +120,21 @@ def test_image_windows_equal_forward(lc):
     y = np.array(Y).reshape(2, nv, order="F")
     ref = np.concatenate([y[0] * np.float32(s.p_wfs.pixsize), y[1] * np.float32(s.p_wfs.pixsize)])
     assert np.array_equal(got, ref.astype(np.float32))
+
+
+def test_noise_free_fused_frame_on_the_fft_method(lc):
+    """The fused learned frame of the FFT method keeps the in-register FFT when
+    noise-free too (the bits that workgroup size 64 names), where comp_image
+    takes the split-FP16 products: the same spots to 1e-6 of the largest pixel
+    (8 units of rounding)."""
+    s = lc.sys
+    slopes = _obj(lc, np.zeros(2 * s.wfs.nvalid))
+    lc.sutra.comp_frame(s.wfs, lc.mlp, slopes, False)
+    fused = s.bincube()
+    alone = []
+    for wg in (64, 0):
+        s.wfs.set_wg_size(wg)
+        s.wfs.comp_image(False)
+        alone.append(s.bincube())
+    assert np.array_equal(fused, alone[0])
+    assert 0.0 < np.abs(fused - alone[1]).max() < 1e-6 * fused.max()
