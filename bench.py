@@ -179,6 +179,19 @@ def measure(method, cfg_name, steps, warmup, phase, thr, wg=0):
     return out, s
 
 
+def tune_launch(b, k, split, frames_per_graph):
+    """The fastest launch grid (workgroups; 0: one per tile) and XCD mapping of
+    a batch of k WFS on the FFT method at one split, kept set."""
+    times = {}
+    for grid in (0, 512, 1024, 2048):
+        for remap in (0, 1):
+            b.set_tiles([0] * k, [split] * k, grid, remap)
+            b.capture(frames_per_graph)
+            b.replay(3)
+            times[grid, remap] = min(b.replay(5) for _ in range(4))
+    b.set_tiles([0] * k, [split] * k, *min(times, key=times.get))
+
+
 def measure_batched(method, k, phase, thr, graphs=10, frames_per_graph=20):
     """k independent 80x80 frames (own screens and outputs) per launch through
     sutra.WfsBatch, replayed from a captured hipGraph."""
@@ -193,11 +206,12 @@ def measure_batched(method, k, phase, thr, graphs=10, frames_per_graph=20):
         systems.append(s)
     import sutra
     b = sutra.WfsBatch(systems[0].ctx, [s.wfs for s in systems], [s.centro for s in systems], False)
-    # split 2: the FFT; 0: the products.  The autotuner (launch grid, XCD mapping)
-    # tries both, so the plain FFT keeps the default grid
-    b.set_tiles([LIBRARY_METHOD[method]] * k, [2 if method == 0 else 0] * k)
-    if method != 0:
-        b.autotune(method_mask=1 << LIBRARY_METHOD[method], reps=10)
+    if LIBRARY_METHOD[method] == 0:
+        # split 2 names the in-register FFT, 0 the products: the autotuner would
+        # try both, so only the launch grid and the XCD mapping are searched
+        tune_launch(b, k, 2 if method == 0 else 0, frames_per_graph)
+    else:
+        b.autotune(method_mask=1 << method, reps=10)
     b.capture(frames_per_graph)
     b.replay(2)
     sync()
