@@ -34,8 +34,11 @@ constexpr int kFftNoisyWaves = 4;
 // that the lanes that idle in the transforms cost as much.  Per frame, N lanes
 // and a wave per sub-aperture: nfft 32, 8x8 px, 40x40 (1,256) 20.4 and 15.5
 // us, 50x50 (1,944) 20.9 and 16.1, 60x60 (2,792) 23.3 and 23.8, 80x80 35.5 and
-// 34.3; nfft 16, 40x40 24.3 and 13.7, 74x74 (4,268) 24.6 and 28.7.  (nfft 64
-// has 64 lanes already.)
+// 34.3; nfft 16, 40x40 24.3 and 13.7, 50x50 25.1 and 14.5, 74x74 (4,268) 24.6
+// and 28.7.  Below the line one wave each was faster at 52 to 1,944
+// sub-apertures, 50 and 1,000 photons, 5 to 12 pixels a side and every binning
+// (1.1 to 1.9 times); nfft 32 crosses before 2,792, nfft 16 before 4,268.  (nfft
+// 64 has 64 lanes already.)
 constexpr int kFftNoisyMax = 2048;
 template <int N, int R>
 __global__ __launch_bounds__(64 * kFftNoisyWaves) __attribute__((amdgpu_waves_per_eu(2)))
@@ -95,13 +98,13 @@ static int32_t launch_fft_nrt(const ImageParams& p, hipStream_t st, BgParams bg)
 
 template <int N, int R>
 static int32_t launch_fft_nr(const ImageParams& p, hipStream_t st, const BgParams& bg) {
-  // workgroup size: 64 lanes by default (more, smaller workgroups spread the
-  // sub-apertures evenly over the 256 CUs); 256 on request (tuning)
   // noisy frames of few sub-apertures: one wave each (kFftNoisyMax)
   if constexpr (N == 16 || N == 32) {
     if (p.tpb == 0 && p.noise > -1.0f && p.nvalid <= kFftNoisyMax)
       return launch_fft_noisy<N, R>(p, st, bg);
   }
+  // workgroup size: 64 lanes by default (more, smaller workgroups spread the
+  // sub-apertures evenly over the 256 CUs); 256 on request (tuning)
   if (p.tpb == 256) return launch_fft_nrt<N, R, 256>(p, st, bg);
   if (p.tpb == 128 && N <= 128) return launch_fft_nrt<N, R, 128>(p, st, bg);
   return launch_fft_nrt<N, R, 64>(p, st, bg);
