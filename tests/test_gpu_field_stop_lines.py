@@ -41,3 +41,30 @@ def test_every_length_matches_oracle(n, npup):
     bar = 4 * 2 * np.log2(n) * 2.0 ** -24 + 4 * 2.0 ** -22  # and the output angle's rounding
     print("  error %.2e (bar %.2e)" % (err, bar), flush=True)
     assert err < bar
+
+
+@pytest.mark.parametrize("n,npup", [(256, 193), (512, 311), (1024, 645), (2048, 1030),
+                                    (4096, 1283)])
+def test_mean_energy_is_kept(n, npup):
+    """An all-pass stop gives the field back: the mean of its squared amplitude
+    over tens of thousands of points, where random roundings cancel, keeps what
+    the rounded twiddles lose or the output scale gives back.  Half a unit of
+    that scale on the amplitude, 2 x 2^-24, and a quarter of that for the
+    twiddles between the passes."""
+    import torch
+    lib = capi.load()
+    rng = np.random.default_rng(n)
+    phase = (2.0 * rng.standard_normal((npup, npup))).astype(np.float32)
+    t = lambda a: torch.tensor(np.ascontiguousarray(a.T.ravel()), device="cuda")
+    d = [t(phase), t(np.ones((npup, npup), np.float32)), t(np.ones((n, n), np.float32))]
+    work = torch.zeros(2 * n * npup, dtype=torch.float32, device="cuda")
+    oph = torch.zeros(npup * npup, dtype=torch.float32, device="cuda")
+    oam = torch.zeros_like(oph)
+    print("all-pass n=%d npup=%d" % (n, npup), flush=True)
+    rc = lib.shwfs_field_stop(capi.ptr(d[0]), capi.ptr(d[1]), npup, 10.0, capi.ptr(d[2]), n,
+                              capi.ptr(work), capi.ptr(oph), capi.ptr(oam), None)
+    assert rc == 0, capi.last_error(lib)
+    torch.cuda.synchronize()
+    gain = float((oam.double() ** 2).mean()) - 1.0
+    print("  energy %.2e" % gain, flush=True)
+    assert abs(gain) < 1.25 * 2.0 ** -23
