@@ -133,3 +133,26 @@ def test_named_workgroup_size_and_noisy_member_take_the_fft():
     g, s = _out(bs)[0], bs.systems[0]
     assert relative_array_error(g[0], _alone(s, 64)[0]) == 0.0
     assert 0.0 < relative_array_error(g[0], _alone(s, 0)[0]) < 1e-6
+
+
+@pytest.mark.parametrize("pd,nfft,nrebin,npix", [(8, 16, 2, 8), (16, 32, 4, 8), (13, 32, 3, 9)])
+def test_noisy_fft_batch_against_the_frame_alone(pd, nfft, nrebin, npix):
+    """The same draws: spots and image equal bit for bit.  Alone the frame runs
+    one wave per sub-aperture and sums its float moments over 64 lanes, in the
+    batch over nfft: a few units of rounding of centroids of up to 9 pixels,
+    5e-6 of the largest slope."""
+    cfgs = [_cfg(nx, pd, nfft, nrebin, npix, seed=nx) for nx in (9, 14)]
+    bs = _batch(cfgs)
+    for k, s in enumerate(bs.systems):
+        s.wfs.set_noise(0.5, 77 + k)
+    bs.batch = bs.sutra.WfsBatch(bs.systems[0].ctx, [s.wfs for s in bs.systems],
+                                 [s.centro for s in bs.systems], True)
+    bs.batch.set_frame(0)
+    got = _out(bs)
+    for k, s in enumerate(bs.systems):
+        s.wfs.set_noise(0.5, 77 + k)  # call counter 0
+        s.sutra.comp_frame(s.wfs, s.centro, s.rtc.d_control[0].d_centroids, True)
+        e = [relative_array_error(a, b)
+             for a, b in zip(got[k], (s.bincube(), s.binimg(), s.slopes()))]
+        print("nvalid %d: spots %.1e image %.1e slopes %.1e" % (s.wfs.nvalid, *e), flush=True)
+        assert e[:2] == [0.0, 0.0] and e[2] < 5e-6
