@@ -90,7 +90,7 @@ int32_t fill_task(shwfs_batch* b, int i, const shwfs_batch_tile& tile, bool prod
   int32_t rc = check_geom(&g, tile.method);
   if (rc) return rc;
   products = products && tile.method == SHWFS_METHOD_FFT_FP32 && tile.split == 0 && !b->noisy &&
-             split_fp16_fits(t.P, nfft);
+             split_fp16_fits(t.P, nfft, false);
   if (tile.method == SHWFS_METHOD_FFT_FP32 && !products) {
     int split = tile.split;
     if (split == 0) split = 2 * pdiam <= nfft ? 2 : 1;

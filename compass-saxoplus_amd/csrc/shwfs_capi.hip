@@ -642,7 +642,7 @@ static int32_t comp_image_on(const shwfs_sh_geom* g, const shwfs_frame_args* f, 
   // and shorter ones: slopes 1-4 % further from float64 although the spots are
   // closer.  Float64 moments end that.
   const bool products = !ext && !mlp && f->method == SHWFS_METHOD_FFT_FP32 &&
-                        split_fp16_fits(p, g->nfft);
+                        split_fp16_fits(p, g->nfft, f->nlayers > 0);
   if (products) p.fp64 = 1;
   if (ext) return launch_image_ext(p, ext_params(g), g->nfft, g->ntot, st);
   if (f->nlayers > 0) {

@@ -60,10 +60,12 @@ int32_t launch_image_dft(const ImageParams& p, int nfft, int method, hipStream_t
   return fail(SHWFS_ERR_ARG, "unknown DFT method");
 }
 
-bool split_fp16_fits(const ImageParams& p, int nfft) {
-  if (p.noise > -1.0f || p.tpb != 0 || p.pdiam > 16) return false;
-  if (nfft == 32) return p.pdiam >= 5;
-  return nfft == 16 && p.pdiam >= (dft_register_rebin(p) > 0 ? 7 : 9);
+bool split_fp16_fits(const ImageParams& p, int nfft, bool traced) {
+  constexpr int kGatherMax = 4096;
+  if (p.noise > -1.0f || p.tpb != 0 || p.pdiam < 5 || p.pdiam > 16) return false;
+  if (nfft == 32) return true;
+  return nfft == 16 &&
+         (p.pdiam > 8 || dft_register_rebin(p) > 0 || p.nvalid <= kGatherMax || traced);
 }
 
 int32_t launch_image_split(const ImageParams& p, int nfft, hipStream_t st) {

@@ -31,14 +31,16 @@
 //     2^-23 |x| while lo is a normal fp16.  The power-of-two scales of FP16 see
 //     to that for the table and G; a unit window's field enters unscaled, so a
 //     lo below 2^-14 is a multiple of 2^-24 and small components are held to
-//     2^-25 absolute, a float's rounding near 1.  (Field and table scaled evenly, 2^6 and 2^4,
-//     and the fourth product lo*lo moved no error against float64 by more than
-//     its spread over screens.)  For nfft 16 and 32 with windows of up to 16
+//     2^-25 absolute, a float's rounding near 1.  (Field and table scaled
+//     evenly, 2^6 and 2^4, and the fourth product lo*lo moved no error against
+//     float64 by more than its spread over screens; the table's lo taken from
+//     float64 halved the flux's.)  For nfft 16 and 32 with windows of up to 16
 //     points.  Relative error of the spots against float64 over those shapes:
-//     6-11e-8, the in-register FP32 FFT's 6-11e-8 (80x80, nfft 32: 7.8e-8
-//     against 8.8e-8; 40x40, nfft 16: 8.5 against 8.9e-8).  The FFT is bound by
-//     its 1,660 VALU instructions per two sub-apertures; here the transform is
-//     on the matrix cores.
+//     6-11e-8, the in-register FP32 FFT's 6-11e-8 (nfft 32, 16 points, 4x4
+//     binning: 7.9e-8 against 9.0e-8; nfft 16, 8 points: 8.0 against 8.8e-8), of
+//     the flux 3-7e-8 against 6-11e-8.  The FFT is bound by its 1,660 VALU
+//     instructions per two sub-apertures; here the transform is on the matrix
+//     cores.
 // Binning, noise, detector image and
 // centroids follow the same definitions as the FFT kernel.
 #pragma once
@@ -216,10 +218,12 @@ struct alignas(16) SplitTable {
           const int idx = (kx * x) % N;
           const double cs = c[idx], sn = c[(idx + N - N / 4) % N];  // cos, sin of 2 pi idx / N
           // [Wr, -Wi; Wi, Wr] with W = cos - i sin
-          const float w = (float)(row_im == col_im ? cs : (row_im ? -sn : sn));
-          const _Float16 h = (_Float16)w;
+          // lo from the float64 value: rounded to float first, cos(pi/4) and its
+          // like end below themselves, and the mean of |w|^2 2.9 to 3.6e-8 low
+          const double w = row_im == col_im ? cs : (row_im ? -sn : sn);
+          const _Float16 h = (_Float16)(float)w;
           v[f][l][0][e] = h;
-          v[f][l][1][e] = (_Float16)(w - (float)h);
+          v[f][l][1][e] = (_Float16)(float)(w - (double)(float)h);
         }
   }
 };

@@ -214,23 +214,24 @@ int32_t launch_image_dft(const ImageParams& p, int nfft, int method, hipStream_t
                          const void* wtab = nullptr, const BgParams& bg = {});
 // Noise-free frames of SHWFS_METHOD_FFT_FP32 on the matrix cores
 // (split-FP16 products of FP32 accuracy, shwfs_image_dft.hpp): whether the
-// frame takes that kernel, and its launch.  The line lies where the products
-// are faster and no further from float64 than the FFT, over 10x10, 40x40 and
-// 80x80, each binning, and 16 to 64 screens:
-//   * nfft 32, windows of 5 to 16 points: 1.05 to 2.2 times faster (80x80, 16
+// frame (traced: through the layers) takes that kernel, and its launch.  The
+// line lies where the products are faster and no further from float64 than the
+// FFT, over 10x10, 40x40 and 80x80, each binning, and 32 screens:
+//   * windows of 5 to 16 points, nfft 32: 1.05 to 2.2 times faster (80x80, 16
 //     points, 4x4 binning 11.4 and 6.9 us a frame, the general binmap of 5
-//     points 10.3 and 9.6); spots 0.9 to 1.02 of the FFT's error, flux 0.75 to
-//     0.9.  Past 16 points the FFT is faster (24 points 12.4 and 26.2; nfft 64,
-//     16 points, 40x40 11.8 and 20.2; 32 points 14.4 and 23.2).
-//   * nfft 16, windows of 7 points with register binning, 9 with the general
-//     binmap: 1.08 to 2.1 times faster; spots 0.9 to 1.01, flux 0.92 to 1.02.
-//     Shorter windows take a half-size FFT of few roundings, which the products
-//     do not reach: flux 1.04 to 1.08 of its error at 5 points, and with the
-//     general binmap 1.03 to 1.05 at 5 to 8, where an 80x80 frame is slower too
-//     (6.8 and 7.0 us).
+//     points 10.3 and 9.6); spots 0.8 to 1.0 of the FFT's error (general binmap
+//     up to 1.05), flux 0.4 to 0.65.  nfft 16: 1.08 to 2.1 times faster; spots
+//     0.83 to 1.0 (general binmap up to 1.03), flux 0.5 to 0.9.
+//   * below 5 points spots come 3 to 10 % further off; past 16 the FFT is faster
+//     (24 points 12.4 and 26.2; nfft 64, 16 points, 40x40 11.8 and 20.2; 32
+//     points 14.4 and 23.2).
+//   * nfft 16, windows of up to 8 points (a half-size FFT), general binmap: up to
+//     4,096 sub-apertures (4,024: 6.5 and 6.3 us; 4,972: 6.7 and 6.9).  Traced
+//     frames are faster with the products past that too, whose layers are read
+//     by rows.
 // A frame that names a workgroup size (wg_size) keeps the in-register FFT, and
 // so does a noisy one: its photon draws would move where a spot's last bit does.
-bool split_fp16_fits(const ImageParams& p, int nfft);
+bool split_fp16_fits(const ImageParams& p, int nfft, bool traced);
 int32_t launch_image_split(const ImageParams& p, int nfft, hipStream_t s);
 int32_t launch_mfma_probe(const float* A, const float* B, float* D, int method, hipStream_t s);
 // img = sigma * N(0,1) (Philox domain `domain`, element = image index); the

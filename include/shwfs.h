@@ -34,10 +34,11 @@ enum {
 enum {
   SHWFS_METHOD_FFT_FP32 = 0,   /* plain FP32: in-register radix-2 FFT; noise-free frames of
                                   the default workgroup size with windows of 5 to 16
-                                  points at nfft 32 or 7 to 16 at nfft 16 (9 to 16 where
-                                  the binning is not a block of 1, 2 or 4 about the
-                                  centre) take split-FP16 products of the same accuracy
-                                  on the matrix cores */
+                                  points at nfft 16 or 32 take split-FP16 products of
+                                  the same accuracy on the matrix cores (but past 4,096
+                                  sub-apertures not windows of up to 8 points at nfft 16
+                                  whose binning is no block of 1, 2 or 4 about the
+                                  centre, untraced) */
   SHWFS_METHOD_DFT_BF16X3 = 1, /* pruned DFT on MFMA, split-BF16x3, FP32 accumulate */
   SHWFS_METHOD_DFT_FP16 = 2    /* pruned DFT on MFMA, FP16 with per-subap scale */
 };

@@ -1,6 +1,5 @@
-"""Noise-free frames of the FFT method: the split-FP16 products (nfft 32,
-windows of 5 to 16 points; nfft 16, 7 to 16, or 9 to 16 with the general
-binmap) against the in-register FFT that a named
+"""Noise-free frames of the FFT method: the split-FP16 products (windows of 5
+to 16 points at nfft 16 and 32) against the in-register FFT that a named
 workgroup size selects, and both against the float64 oracle, over every form
 that the products take: each rebin code, the general binmap (nrebin 3), full
 and small windows, one sub-aperture to several workgroups, amplitudes far from
@@ -107,30 +106,37 @@ def test_named_workgroup_size_keeps_the_fft():
     assert 0.0 < relative_array_error(got[3], got[0]) < 1e-6
 
 
-@pytest.mark.parametrize("pd,nfft,nrebin,npix,products", [
-    (6, 16, 2, 8, False), (7, 16, 2, 8, True), (16, 16, 1, 10, True), (8, 16, 3, 5, False),
-    (9, 16, 3, 5, True), (8, 16, 2, 7, False), (9, 16, 2, 7, True), (4, 32, 4, 8, False),
-    (5, 32, 4, 8, True), (5, 32, 3, 9, True), (16, 32, 2, 11, True), (17, 32, 4, 8, False),
-    (16, 64, 4, 8, False)])
-def test_forms_that_take_the_products(pd, nfft, nrebin, npix, products):
-    """Which frames are the FFT's own bits, on both sides of each edge (2x2
-    binning of 7 pixels starts off the block grid: the general binmap)."""
-    s, _ = _system(12, pd, nfft, nrebin, npix)
+@pytest.mark.parametrize("nx,pd,nfft,nrebin,npix,products", [
+    (12, 4, 16, 2, 8, False), (12, 5, 16, 2, 8, True), (12, 16, 16, 1, 10, True),
+    (12, 8, 16, 3, 5, True), (12, 8, 16, 2, 7, True), (72, 8, 16, 3, 5, True),
+    (76, 8, 16, 3, 5, False), (76, 9, 16, 3, 5, True), (76, 8, 16, 2, 8, True),
+    (12, 4, 32, 4, 8, False), (12, 5, 32, 4, 8, True), (12, 5, 32, 3, 9, True),
+    (12, 16, 32, 2, 11, True), (12, 17, 32, 4, 8, False), (12, 16, 64, 4, 8, False)])
+def test_forms_that_take_the_products(nx, pd, nfft, nrebin, npix, products):
+    """Which frames are the FFT's own bits, on both sides of each edge: windows
+    of 5 and 16 points, and at nfft 16 windows of 8 points with the general
+    binmap (nrebin 3; 2x2 binning of 7 pixels starts off the block grid) at 4,096
+    sub-apertures (72x72: 4,024; 76x76: 4,488)."""
+    s, _ = _system(nx, pd, nfft, nrebin, npix)
     fft, default = _both(s)
     e = relative_array_error(default[0], fft[0])
-    print("pd %d nfft %d nrebin %d npix %d: %.1e" % (pd, nfft, nrebin, npix, e), flush=True)
+    print("nvalid %d pd %d nfft %d nrebin %d npix %d: %.1e"
+          % (s.wfs.nvalid, pd, nfft, nrebin, npix, e), flush=True)
     assert (0.0 < e < 1e-6) if products else all(np.array_equal(a, b)
                                                  for a, b in zip(fft, default))
 
 
-@pytest.mark.parametrize("pd,nfft,nrebin,npix", [
-    (7, 16, 2, 8), (8, 16, 2, 8), (16, 16, 2, 8), (11, 16, 3, 5), (5, 32, 4, 8), (8, 32, 3, 9),
-    (11, 32, 3, 9), (16, 32, 2, 12), (16, 32, 4, 8)])
-def test_products_are_no_further_off_than_the_fft(pd, nfft, nrebin, npix):
+@pytest.mark.parametrize("pd,nfft,nrebin,npix,spots", [
+    (5, 16, 1, 10, 1.05), (5, 16, 2, 8, 1.05), (8, 16, 2, 8, 1.05), (8, 16, 3, 5, 1.1),
+    (16, 16, 2, 8, 1.05), (11, 16, 3, 5, 1.1), (5, 32, 4, 8, 1.05), (8, 32, 3, 9, 1.1),
+    (11, 32, 3, 9, 1.1), (16, 32, 2, 12, 1.05), (16, 32, 4, 8, 1.05)])
+def test_products_are_no_further_off_than_the_fft(pd, nfft, nrebin, npix, spots):
     """Relative error (2-norm) of spots and flux against the oracle, the mean
     over 16 screens.  The two errors are of independent roundings: their ratio
     spreads by 7 % from screen to screen (some 100 sub-apertures each), 1.8 %
-    over 16, so the products' is at most 1.05 times the FFT's."""
+    over 16.  Spots: at most 1.05 times the FFT's, 1.1 with the general binmap
+    (0.8 to 1.0 and 0.97 to 1.05 over 32 other screens).  Flux: 0.95 (0.4 to 0.9;
+    its mean error, which the table's rounding sets, is most of it)."""
     nx = 12
     c = configs.sh_config(0.2 * nx, nx, pd, npix, nfft, nrebin, nphot=1000.0,
                           seeds=range(1, 17))
@@ -144,4 +150,4 @@ def test_products_are_no_further_off_than_the_fft(pd, nfft, nrebin, npix):
                 err[k, q] += np.linalg.norm(g.astype(np.float64) - w) / np.linalg.norm(w) / 16
     print("pd %d nfft %d nrebin %d: spots %.3e %.3e flux %.3e %.3e"
           % (pd, nfft, nrebin, err[0, 0], err[1, 0], err[0, 1], err[1, 1]), flush=True)
-    assert np.all(err[1] <= 1.05 * err[0])
+    assert err[1, 0] <= spots * err[0, 0] and err[1, 1] <= 0.95 * err[0, 1]
